@@ -16,6 +16,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <future>
 #include <mutex>
 #include <new>
 #include <numeric>
@@ -162,7 +163,8 @@ struct mfcfd_ctx {
         DevBuf<int> seq, old_pts, old_src, wait_src;
         DevBuf<long long> take_ptr;
         DevBuf<unsigned> take;
-        DevBuf<unsigned char> late;
+        DevBuf<unsigned char> late, late_src;
+        DevBuf<int> slots;
         DevBuf<double> wgt;
         std::vector<int> level_ptr;   // host copy of the level cuts of seq
         int count = 0;
@@ -174,6 +176,8 @@ struct mfcfd_ctx {
             take_ptr.release();
             take.release();
             late.release();
+            late_src.release();
+            slots.release();
             wgt.release();
             level_ptr.clear();
             count = 0;
@@ -210,6 +214,7 @@ struct mfcfd_ctx {
     hipGraphExec_t graph_exec = nullptr;
     bool graph_stale = true;
     int sweep_grid = 0, sweep_grid_mixed = 0;
+    int sweep_chain[2] = {1, 1};   // longest chain of the sweep groups, by precision
     // bookkeeping of fpi_solver.f90:38-43
     double res_old = 0.0, res_new = 0.0, residue = 0.0, max_res = 0.0, sum_res_sqr = 0.0;
     int max_res_point = 0, last_t = 0;
@@ -426,6 +431,9 @@ SweepAsync sweep_args(mfcfd_ctx* c, mfcfd_ctx::DevSweepDir& d) {
     a.take_ptr = d.take_ptr.p;
     a.take = d.take.p;
     a.late = d.late.p;
+    a.slots = d.slots.p;
+    a.late_src = d.late_src.p;
+    a.groups = (int)(d.slots.n / kSweepGroup);
     a.wgt = d.wgt.p;
     a.old_pts = d.old_pts.p;
     a.n_old = (int)d.old_pts.n;
@@ -441,6 +449,7 @@ SweepAsync sweep_args(mfcfd_ctx* c, mfcfd_ctx::DevSweepDir& d) {
     a.ctr = c->sweep_ctr.p;
     a.stalls = &c->rec.p->stalls;
     a.zero = 0;
+    a.split = c->sweep_chain[c->fp.mixed] > 1;
     return a;
 }
 
@@ -491,6 +500,22 @@ int do_sweeps(mfcfd_ctx* c) {
     return launch_error("implicit sweeps");
 }
 
+// Longest chain of positions a sweep workgroup hands from wave to wave, from
+// the waves resident on the chip and the plan's mean positions per dependency
+// level.  A chain shortens the path through the levels, and holds all eight
+// waves of its workgroup until its last position is done: with many levels in
+// flight that costs nothing, with few it keeps ready positions waiting.  Sweep
+// kernel times, in ms, with chains of 1 (late entries not set apart), 2 and 8:
+//   1M FP64, 13.6 levels in flight    11.4   9.7   9.2
+//   3M FP64, 6.8                      20.5  18.0  18.9
+//   8M FP64, 4.1                      33.8  35.4  41.5
+//   3M mixed, 13.6                    17.5  13.4  12.9
+//   8M mixed, 8.2                     26.8  22.5  23.5
+int chain_for(int resident_waves, double per_level) {
+    const double levels = resident_waves / std::max(per_level, 1.0);
+    return levels >= 12.0 ? kSweepGroup : levels >= 6.0 ? 2 : 1;
+}
+
 // Builds the LU-SGS plan of the given implicit form (SweepPlan) from the
 // host copies kept at bind, uploads it and computes every entry's weight.
 // Synchronous; never called while a graph is being captured.
@@ -531,6 +556,15 @@ int build_plan(mfcfd_ctx* c, int form) {
     }
     SweepPlan plan;
     if (plan.build(in)) return fail(MFCFD_EINVAL, "sweep plan: a dependency does not precede its point");
+    const int resident[2] = {kSweepGroup * sweep_async_grid(n, c->params.power == 0.0, false),
+                             kSweepGroup * sweep_async_grid(n, c->params.power == 0.0, true)};
+    const double per_level = 2.0 * (double)plan.fwd.seq.size() /
+                             std::max<double>(1.0, (double)(plan.fwd.level_ptr.size() + plan.bwd.level_ptr.size()) - 2.0);
+    for (int m = 0; m < 2; ++m) c->sweep_chain[m] = chain_for(resident[m], per_level);
+    const int chain = c->sweep_chain[c->fp.mixed];
+    std::future<void> f = std::async([&] { group_positions(plan.fwd, n, chain); });
+    group_positions(plan.bwd, n, chain);
+    f.get();
     hipStream_t st = c->stream;
     c->sw_fwd.release();
     c->sw_bwd.release();
@@ -550,6 +584,10 @@ int build_plan(mfcfd_ctx* c, int form) {
         const unsigned char none_c = 0;
         if ((r = upload(d.late, pd.late.empty() ? &none_c : pd.late.data(), std::max<size_t>(pd.late.size(), 1), st)))
             return r;
+        if ((r = upload(d.late_src, pd.late_src.empty() ? &none_c : pd.late_src.data(),
+                        std::max<size_t>(pd.late_src.size(), 1), st)))
+            return r;
+        if ((r = upload(d.slots, pd.slots.data(), pd.slots.size(), st))) return r;
         if (d.wgt.alloc(std::max<size_t>(pd.take.size(), 1)) != hipSuccess)
             return fail(MFCFD_ENOMEM, "sweep weights (%zu entries)", pd.take.size());
         if ((r = upload(d.old_pts, pd.old_pts.data(), pd.old_pts.size(), st))) return r;
@@ -559,7 +597,7 @@ int build_plan(mfcfd_ctx* c, int form) {
     };
     if ((rc = put(c->sw_fwd, plan.fwd))) return rc;
     if ((rc = put(c->sw_bwd, plan.bwd))) return rc;
-    if (c->pub.n == 0 && c->pub.alloc_fine(5ULL * n) != hipSuccess)
+    if (c->pub.n == 0 && c->pub.alloc_fine(8ULL * n) != hipSuccess)
         return fail(MFCFD_ENOMEM, "sweep values (fine-grained)");
     // copy sources read as this sweep's delU: a slot each in dsrc
     const size_t n_src = std::max(plan.fwd.wait_src.size(), plan.bwd.wait_src.size());
@@ -586,8 +624,9 @@ int build_plan(mfcfd_ctx* c, int form) {
     launch_sweep_weights(c->geom(), sweep_args(c, c->sw_bwd), c->fp.power, st);
     if ((rc = launch_error("sweep weights"))) return rc;
     HIP_TRY(hipStreamSynchronize(st));   // the host plan ends here
-    c->sweep_grid = sweep_async_grid(c->sw_fwd.count, c->params.power == 0.0, false);
-    c->sweep_grid_mixed = sweep_async_grid(c->sw_fwd.count, c->params.power == 0.0, true);
+    const int groups = (int)(std::max(plan.fwd.slots.size(), plan.bwd.slots.size()) / kSweepGroup);
+    c->sweep_grid = sweep_async_grid(groups, c->params.power == 0.0, false);
+    c->sweep_grid_mixed = sweep_async_grid(groups, c->params.power == 0.0, true);
     c->plan_form = form;
     c->graph_stale = true;
     return MFCFD_OK;

@@ -60,6 +60,13 @@ struct SweepAsync {
     const unsigned* take;       // k << 4 | wait << 3 | direction (7: supersonic copy) of every taken entry
     const unsigned char* late;  // [count]: position t's last late[t] entries read the wait dependency
                                 // that executes last (at most 4; 0: none set apart)
+    const int* slots;           // [kSweepGroup*groups] position of each wave of a group (-1: none); not
+                                // read when split is 0
+    const unsigned char* late_src;  // [count]: 1 + the wave of the same group that executes the point of
+                                // position t's late entries, 0: another group's
+    int groups;
+    int split;                  // 1: groups of chains, late entries summed after the others; 0: groups of
+                                // consecutive positions, every entry waited for together (same sums)
     double* wgt;                // [entries] least-squares weight of each entry (set at bind)
     const int* old_pts;         // points some entry reads as old: pold is taken for them
     int n_old;
@@ -127,7 +134,7 @@ void launch_sweeps_levels(const DevGeom& g, const DevState& s, const FlowParams&
 void launch_sweeps_async(const DevGeom& g, const DevState& s, const FlowParams& p, const SweepAsync& fwd,
                          const SweepAsync& bwd, int grid, hipStream_t st, const hipEvent_t* ev = nullptr);
 // resident workgroup count used for the sync-free sweeps
-int sweep_async_grid(int count, bool unit_weight, bool mixed);
+int sweep_async_grid(int groups, bool unit_weight, bool mixed);
 // setup: the least-squares weight of every entry of a sweep's plan
 void launch_sweep_weights(const DevGeom& g, const SweepAsync& a, double power, hipStream_t st);
 // state_update.f90 (+ residual reduction into *rec; hist may be null)

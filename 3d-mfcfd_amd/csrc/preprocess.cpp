@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <future>
 
 namespace mfcfd {
 
@@ -247,12 +248,55 @@ int build_dir(const SweepPlanInputs& in, bool forward, SweepDirPlan& out) {
 
 }  // namespace
 
+void group_positions(SweepDirPlan& plan, int n, int max_chain) {
+    const int m = (int)plan.seq.size();
+    plan.slots.clear();
+    plan.late_src.assign(m, 0);
+    std::vector<int> at(n, -1);
+    for (int u = 0; u < m; ++u) at[plan.seq[u]] = u;
+    // height: the longest chain of dependents below a position; joins: the
+    // candidate of greatest height among those whose late dependency it is
+    std::vector<int> height(m, 0), joins(m, -1);
+    for (int u = m - 1; u >= 0; --u)
+        for (long long e = plan.take_ptr[u]; e < plan.take_ptr[u + 1]; ++e)
+            if (plan.take[e] & kTakeWait) {
+                int& h = height[at[plan.take[e] >> kTakeShift]];
+                h = std::max(h, height[u] + 1);
+            }
+    for (int u = 0; u < m; ++u) {
+        if (!plan.late[u]) continue;
+        int& j = joins[at[plan.take[plan.take_ptr[u + 1] - 1] >> kTakeShift]];
+        if (j < 0 || height[u] > height[j]) j = u;
+    }
+    std::vector<char> placed(m, 0);
+    plan.slots.reserve((size_t)m + kSweepGroup);
+    for (int u = 0; u < m; ++u) {
+        if (placed[u]) continue;
+        placed[u] = 1;
+        plan.slots.push_back(u);
+        for (int tail = u, len = 1; len < max_chain && plan.slots.size() % kSweepGroup != 0; ++len) {
+            const int v = joins[tail];
+            if (v < 0) break;
+            bool ready = true;
+            for (long long e = plan.take_ptr[v]; e < plan.take_ptr[v + 1] && ready; ++e)
+                if (plan.take[e] & kTakeWait) ready = placed[at[plan.take[e] >> kTakeShift]];
+            if (!ready) break;
+            placed[v] = 1;
+            plan.late_src[v] = (unsigned char)(1 + (plan.slots.size() - 1) % kSweepGroup);
+            plan.slots.push_back(v);
+            tail = v;
+        }
+    }
+    while (plan.slots.size() % kSweepGroup != 0) plan.slots.push_back(-1);
+}
+
 int SweepPlan::build(const SweepPlanInputs& in) {
     backup = in.backup;
     n_visited = (int)in.visit_fwd.size();
-    if (build_dir(in, true, fwd)) return -1;
-    if (build_dir(in, false, bwd)) return -1;
-    return 0;
+    // the two directions side by side (on one thread where no other is to be had)
+    std::future<int> f = std::async([&] { return build_dir(in, true, fwd); });
+    const int b = build_dir(in, false, bwd);
+    return f.get() || b ? -1 : 0;
 }
 
 }  // namespace mfcfd

@@ -42,6 +42,9 @@ struct SweepDirPlan {
     std::vector<unsigned> take;       // k << 4 | wait << 3 | direction (kTakeCopy: copy entry)
     std::vector<unsigned char> late;  // per position: its last entries, which read the wait
                                       // dependency that executes last (0..kMaxLate; 0: none)
+    std::vector<int> slots;           // group g's wave w executes position slots[kSweepGroup*g + w] (-1: none)
+    std::vector<unsigned char> late_src;  // per position: 1 + the wave that executes its late entries'
+                                      // point when that is in the same group, else 0
     std::vector<int> old_pts;         // points some regular entry reads as old
     std::vector<int> old_src;         // copy sources read as old
     std::vector<int> wait_src;        // copy sources read as this sweep's value
@@ -51,6 +54,8 @@ constexpr unsigned kTakeWait = 8u;
 // at most this many entries of a position are set apart as late (one lane each)
 constexpr int kMaxLate = 4;
 constexpr unsigned kTakeCopy = 7u;
+// positions of a group: one per wave of the sweep kernel's workgroup
+constexpr int kSweepGroup = 8;
 constexpr int kTakeShift = 4;
 
 struct SweepPlanInputs {
@@ -79,6 +84,21 @@ struct SweepPlan {
     // checked anyway because the sync-free sweep relies on it)
     int build(const SweepPlanInputs& in);
 };
+
+// Cuts the positions of a built direction into groups of kSweepGroup, which
+// the sweep kernel's workgroups take in order, one position per wave (slots,
+// late_src).  A position whose late dependency's group still has a free wave
+// joins that group, up to max_chain positions in a row: the value then goes
+// from wave to wave through LDS instead of through memory.  Of a position's
+// candidates the one with the longest chain of dependents below it joins.
+//
+// Every position's dependencies lie in its own group or in earlier ones: a
+// position starts a chain only when every position before it has a group, and
+// joins one only when all of its dependencies have.  The lowest unfinished
+// group therefore never waits for a later one, and inside it positions wait
+// only for earlier positions, so groups taken in order always finish,
+// however few of them run at a time.
+void group_positions(SweepDirPlan& plan, int n, int max_chain);
 
 // the list a sweep walks for point i and direction d (device numbers):
 // the flux stencil's list, except that a wall point takes no ZPOS term and
