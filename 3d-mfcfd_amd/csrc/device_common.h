@@ -16,18 +16,17 @@ inline int grid_for(long long n, int block) { return (int)((n + block - 1) / blo
 // L2.  Gather kernels renumber their blocks so that every XCD walks one
 // contiguous eighth of the (Morton-ordered) points: a point's neighbours are
 // then mostly read through the same L2.  The map is a bijection of
-// [0, gridDim.x) for any grid size.
+// the nb blocks for any nb.
 constexpr int kXcds = 8;
 
-__device__ __forceinline__ int xcd_block() {
-    const int nb = (int)gridDim.x;
-    const int b = (int)blockIdx.x;
+__device__ __forceinline__ int xcd_block(int b, int nb) {
     const int x = b % kXcds, r = b / kXcds;
     const int q = nb / kXcds, rem = nb % kXcds;
     return x * q + (x < rem ? x : rem) + r;
 }
 
 // index of this thread when the launch covers count items, blocks renumbered per XCD
+__device__ __forceinline__ int xcd_block() { return xcd_block((int)blockIdx.x, (int)gridDim.x); }
 __device__ __forceinline__ int xcd_index() { return xcd_block() * (int)blockDim.x + (int)threadIdx.x; }
 
 // The value of v in the lane whose index differs in bit O.  Within aligned
@@ -64,6 +63,36 @@ __device__ __forceinline__ V group_sum(V v) {
     } else {
         return v;
     }
+}
+
+// The value of v in the lane O further on within an aligned group of 4, 8, 16
+// or 32 lanes, all of them active; what the group's last O lanes receive is
+// not used.  Up to 12 a DPP row shift, further through the LDS crossbar.
+template <int O>
+__device__ __forceinline__ int lane_after_b32(int v) {
+    if constexpr (O == 0) return v;
+    else if constexpr (O < 16) return __builtin_amdgcn_update_dpp(v, v, 0x100 | O, 0xf, 0xf, false);
+    else return __shfl_down(v, O, 32);
+}
+template <int O, typename V>
+__device__ __forceinline__ V lane_after(V v) {
+    if constexpr (sizeof(V) == 8) {
+        const long long b = __builtin_bit_cast(long long, v);
+        const int lo = lane_after_b32<O>((int)b), hi = lane_after_b32<O>((int)(b >> 32));
+        return __builtin_bit_cast(V, ((long long)hi << 32) | (long long)(unsigned)lo);
+    } else {
+        return __builtin_bit_cast(V, lane_after_b32<O>(__builtin_bit_cast(int, v)));
+    }
+}
+
+// Adds the terms of a group's G entries to the four running sums its first
+// four lanes hold: lane l adds those of lanes l, l + 4, l + 8, ... in turn.
+// A point's entries l, l + 4, ... thus enter sum l in the same order for every
+// G, and the sums do not depend on how many lanes share the point.
+template <int G, int O = 0, typename V>
+__device__ __forceinline__ V add_terms(V acc, V term) {
+    if constexpr (O < G) return add_terms<G, O + 4>(acc + lane_after<O>(term), term);
+    else return acc;
 }
 
 // group maximum / minimum with the comparisons of a sequential scan

@@ -30,7 +30,8 @@ struct KernelShape {
     int waves = 0;
     int lds = 0;   // dynamic LDS bytes reserved per block: caps the blocks resident per CU
 };
-// shapes the autotuner chooses (defaults until it runs)
+// shapes the autotuner chooses (defaults until it runs); the flux shapes are
+// those of a launch per class (flux_small in kernels_flux_fused.hip)
 struct LaunchShapes {
     KernelShape flux_interior, flux_wall, qderiv;
     int sweep_div = 1;   // sync-free sweeps use the resident grid / sweep_div

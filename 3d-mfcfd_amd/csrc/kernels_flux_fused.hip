@@ -16,9 +16,10 @@
 // (sum_j (G_k - G_i)*(c . (dels, delt, deln)) instead of the 3x3 solve of the
 // accumulated sums), which changes the rounding, not the mathematics.
 //
-// A point is handled by a group of kFluxGroup lanes, each taking every
-// kFluxGroup-th neighbour, and the group sums its partial residuals at the
-// end.  Per lane this is the same work as one lane per point, but a resident
+// A point is handled by a group of lanes, kFluxGroup = 4 of them unless the
+// points are few (flux_small), each taking every fourth neighbour, and the
+// group sums its partial residuals at the end, in an order that does not
+// depend on the number of lanes.  Per lane this is the same work as one lane per point, but a resident
 // wave holds 64 / kFluxGroup points instead of 64: the neighbour data of all
 // points in flight on one XCD then fits its 4 MB L2.  With one lane per point
 // at the 8 resident waves per CU the FP64 kernel's registers allow, each
@@ -213,15 +214,11 @@ __device__ __forceinline__ void octant_axis(const EndState<T>& ei, const EndStat
 // weights and the sums stay FP64.
 // WAVES: minimum waves per SIMD the kernel is compiled for (its register
 // cap); the launch picks one of the compiled variants and a block size
-template <int CLASS, bool UW, typename T, int WAVES>
-__global__ void __launch_bounds__(kBlock, WAVES) k_flux_fused(DevGeom g, DevState s, FlowParams fp, const int* idx,
-                                                             int count) {
-    const unsigned t = (unsigned)xcd_index();
-    const int m = (int)(t / kFluxGroup);
-    const int lane = (int)(t % kFluxGroup);
-    if (m >= count) return;  // whole groups: blocks hold a multiple of kFluxGroup lanes
+// G: lanes that share the point (lane: this one's number among them)
+template <int CLASS, bool UW, typename T, int G>
+__device__ __forceinline__ void flux_point(const DevGeom& g, const DevState& s, const FlowParams& fp, int i,
+                                           int lane) {
     const QArrays<T> qa = qarrays<T>(s);
-    const int i = idx[m];
     const Frame<double> f = load_frame(g.frame, i);
     const Frame<T> ft = frame_as<T>(f);
     const T pi = T(fp.pi);
@@ -240,54 +237,102 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_flux_fused(DevGeom g, DevStat
     const int st_i = CLASS == 1 ? g.status[i] : 0;
     const T sn = st_i == 2 ? T(1) : T(-1);
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int j = lane; j < nb; j += kFluxGroup) {
-        const unsigned e = wk[j];
+    for (int base = 0; base < nb; base += G) {
+        const int j = base + lane;
+        // the entry's own sum over its lists first: it is what add_terms moves
+        double sum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        const unsigned e = j < nb ? wk[j] : 0u;
         const unsigned bits = e & ((1u << kWalkMaskBits) - 1u);
-        if (bits == 0u) continue;
-        const int k = (int)(e >> kWalkMaskBits);
-        const double4 pk = g.pos[k];
-        const double delx = pk.x - pi4.x;
-        const double dely = pk.y - pi4.y;
-        const double delz = pk.z - pi4.z;
-        const double dels = delx * f.t1[0] + dely * f.t1[1] + delz * f.t1[2];
-        const double delt = delx * f.t2[0] + dely * f.t2[1] + delz * f.t2[2];
-        const double deln = delx * f.n[0] + dely * f.n[1] + delz * f.n[2];
-        const double wgt = wls_weight<UW>(dels, delt, deln, fp.power);
-        T prim[5], qi[5];
+        if (bits != 0u) {
+            const int k = (int)(e >> kWalkMaskBits);
+            const double4 pk = g.pos[k];
+            const double delx = pk.x - pi4.x;
+            const double dely = pk.y - pi4.y;
+            const double delz = pk.z - pi4.z;
+            const double dels = delx * f.t1[0] + dely * f.t1[1] + delz * f.t1[2];
+            const double delt = delx * f.t2[0] + dely * f.t2[1] + delz * f.t2[2];
+            const double deln = delx * f.n[0] + dely * f.n[1] + delz * f.n[2];
+            const double wgt = wls_weight<UW>(dels, delt, deln, fp.power);
+            T prim[5], qi[5];
 #pragma unroll
-        for (int r = 0; r < 5; ++r) qi[r] = qip[r];
-        reconstruct_end<T>(qi, dqi, qmi, epsi2_i, T(delx), T(dely), T(delz), prim);
-        const EndState<T> ei = end_state(prim, ft, pi);
-        T qk[5];
+            for (int r = 0; r < 5; ++r) qi[r] = qip[r];
+            reconstruct_end<T>(qi, dqi, qmi, epsi2_i, T(delx), T(dely), T(delz), prim);
+            const EndState<T> ei = end_state(prim, ft, pi);
+            T qk[5];
 #pragma unroll
-        for (int r = 0; r < 5; ++r) qk[r] = qa.qp(k)[r];
-        reconstruct_end<T>(qk, qa.dqp(k), qa.qmp(k), T(limiter_epsi2(fp.vl_const, pk.w)), T(delx), T(dely), T(delz),
-                           prim);
-        const EndState<T> ek = end_state(prim, ft, pi);
-        if (CLASS == 0) {
-            interior_axis<0>(ei, ek, bits, cf, wgt, dels, delt, deln, acc);
-            interior_axis<1>(ei, ek, bits, cf, wgt, dels, delt, deln, acc);
-            interior_axis<2>(ei, ek, bits, cf, wgt, dels, delt, deln, acc);
-        } else {
-            T B3i, er3i, B3k, er3k;
-            axis_terms<2>(ei, B3i, er3i);
-            axis_terms<2>(ek, B3k, er3k);
-            if (st_i == 0) {
-                half_axes_xy(ei, ek, bits, cf, wgt, dels, delt, deln, acc);
+            for (int r = 0; r < 5; ++r) qk[r] = qa.qp(k)[r];
+            reconstruct_end<T>(qk, qa.dqp(k), qa.qmp(k), T(limiter_epsi2(fp.vl_const, pk.w)), T(delx), T(dely),
+                               T(delz), prim);
+            const EndState<T> ek = end_state(prim, ft, pi);
+            if (CLASS == 0) {
+                interior_axis<0>(ei, ek, bits, cf, wgt, dels, delt, deln, sum);
+                interior_axis<1>(ei, ek, bits, cf, wgt, dels, delt, deln, sum);
+                interior_axis<2>(ei, ek, bits, cf, wgt, dels, delt, deln, sum);
             } else {
-                octant_axis<0>(ei, ek, bits, sn, B3i, er3i, B3k, er3k, cf, wgt, dels, delt, deln, acc);
-                octant_axis<1>(ei, ek, bits, sn, B3i, er3i, B3k, er3k, cf, wgt, dels, delt, deln, acc);
+                T B3i, er3i, B3k, er3k;
+                axis_terms<2>(ei, B3i, er3i);
+                axis_terms<2>(ek, B3k, er3k);
+                if (st_i == 0) {
+                    half_axes_xy(ei, ek, bits, cf, wgt, dels, delt, deln, sum);
+                } else {
+                    octant_axis<0>(ei, ek, bits, sn, B3i, er3i, B3k, er3k, cf, wgt, dels, delt, deln, sum);
+                    octant_axis<1>(ei, ek, bits, sn, B3i, er3i, B3k, er3k, cf, wgt, dels, delt, deln, sum);
+                }
+                const unsigned abz = (bits >> (2 * 2)) & 3u;
+                if (abz) half_axis<2>(ei, ek, abz, B3i, er3i, B3k, er3k, cf, wgt, dels, delt, deln, sum);
             }
-            const unsigned abz = (bits >> (2 * 2)) & 3u;
-            if (abz) half_axis<2>(ei, ek, abz, B3i, er3i, B3k, er3k, cf, wgt, dels, delt, deln, acc);
         }
+#pragma unroll
+        for (int r = 0; r < 5; ++r) acc[r] = add_terms<G>(acc[r], sum[r]);
     }
 #pragma unroll
-    for (int r = 0; r < 5; ++r) acc[r] = group_sum<kFluxGroup>(acc[r]);
+    for (int r = 0; r < 5; ++r) acc[r] = group_sum<4>(acc[r]);
     if (lane == 0) {
 #pragma unroll
         for (int r = 0; r < 5; ++r) s.flux_res[5 * (long long)i + r] = st_i == 1 ? 2.0 * acc[r] : acc[r];
     }
+}
+
+template <int CLASS, bool UW, typename T, int WAVES>
+__global__ void __launch_bounds__(kBlock, WAVES) k_flux_fused(DevGeom g, DevState s, FlowParams fp, const int* idx,
+                                                             int count) {
+    const unsigned t = (unsigned)xcd_index();
+    const int m = (int)(t / kFluxGroup);
+    if (m >= count) return;  // whole groups: blocks hold a multiple of kFluxGroup lanes
+    flux_point<CLASS, UW, T, kFluxGroup>(g, s, fp, idx[m], (int)(t % kFluxGroup));
+}
+
+// blocks of the general class in k_flux_small, a whole number per XCD
+__host__ __device__ inline int small_blocks(int points, int lanes) {
+    const int blocks = (int)(((long long)points * lanes + kBlock - 1) / kBlock);
+    return (blocks + kXcds - 1) / kXcds * kXcds;
+}
+
+// Both classes of a cloud that does not fill the chip in one launch, GG lanes
+// per point of the general class, whose points take longer and come first,
+// and GI per point of the interior one, from the next block on.
+template <bool UW, typename T, int GG, int GI>
+__global__ void __launch_bounds__(kBlock, GI == kFluxGroup ? 3 : 2)
+    k_flux_small(DevGeom g, DevState s, FlowParams fp, const int* general, int n_general, const int* interior,
+                 int n_interior) {
+    const int first = small_blocks(n_general, GG), b = (int)blockIdx.x;
+    if (b < first) {
+        const int t = xcd_block(b, first) * kBlock + (int)threadIdx.x, m = t / GG;
+        if (m < n_general) flux_point<1, UW, T, GG>(g, s, fp, general[m], t % GG);   // whole groups
+    } else {
+        const int t = xcd_block(b - first, (int)gridDim.x - first) * kBlock + (int)threadIdx.x, m = t / GI;
+        if (m < n_interior) flux_point<0, UW, T, GI>(g, s, fp, interior[m], t % GI);
+    }
+}
+
+template <bool UW, typename T, int GG, int GI>
+void launch_small(const DevGeom& g, const DevState& s, const FlowParams& p, const TypeLists& tl, int parts,
+                  hipStream_t st) {
+    const int ng = parts & 2 ? tl.n_fused_wall : 0, ni = parts & 1 ? tl.n_fused_interior : 0;
+    const int blocks = small_blocks(ng, GG) + grid_for((long long)ni * GI, kBlock);
+    if (blocks > 0)
+        hipLaunchKernelGGL((k_flux_small<UW, T, GG, GI>), dim3(blocks), dim3(kBlock), 0, st, g, s, p, tl.fused_wall,
+                           ng, tl.fused_interior, ni);
 }
 
 template <int CLASS, typename T>
@@ -323,20 +368,59 @@ void launch_class(const DevGeom& g, const DevState& s, const FlowParams& p, cons
 
 }  // namespace
 
+// Launches both classes together where they do not fill the chip; false: they
+// take a launch each.  Four lanes take a point's 25 neighbours in seven steps
+// of some 7 us (FP64) each when a wave has its SIMD to itself, so with few
+// points the steps are what counts and more lanes share a point: 32 take one
+// step, 16 two.  They cost nothing while the chip has room, about a third more
+// than four lanes once it is full (the lanes beyond 25 idle, terms are moved
+// between lanes).  And the general class, an eighth of the points, leaves the
+// chip mostly idle by itself up to some 100,000 points, so it shares the
+// interior class's launch, until the interior class's registers (four waves
+// per SIMD in FP32 alone, three together) weigh more.  An iteration, in us,
+// before and after:
+//     1,090 points, FP64   142 ->  41     mixed   97 ->  34   (32 + 32 lanes)
+//    20,000                176 ->  89            114 ->  56   (32 + 16)
+//    50,000                204 -> 143            133 ->  91   (16 + 4)
+//   150,000                384 -> 336            229 -> 205   (4 + 4)
+//   500,000               1120 -> 1057           635 -> 625   (4 + 4)
+//   1,000,000 together    2197 -> 2132          1262 -> 1289: a launch each
+template <typename T>
+static bool flux_small(const DevGeom& g, const DevState& s, const FlowParams& p, const TypeLists& tl,
+                       hipStream_t st, int parts) {
+    const int ng = tl.n_fused_wall, ni = tl.n_fused_interior;
+    if (ng > 100000 || ni > 450000) return false;
+    if (p.power != 0.0) {
+        // weighted least squares: the two that cover most sizes
+        if (ng > 20000) return false;
+        if (ni > 24000) launch_small<false, T, 16, 4>(g, s, p, tl, parts, st);
+        else launch_small<false, T, 16, 16>(g, s, p, tl, parts, st);
+    } else if (ng > 20000) {
+        launch_small<true, T, 4, 4>(g, s, p, tl, parts, st);
+    } else if (ni > 24000) {
+        launch_small<true, T, 16, 4>(g, s, p, tl, parts, st);
+    } else if (ng > 4000) {
+        launch_small<true, T, 16, 16>(g, s, p, tl, parts, st);
+    } else if (ni > 4000) {
+        launch_small<true, T, 32, 16>(g, s, p, tl, parts, st);
+    } else {
+        launch_small<true, T, 32, 32>(g, s, p, tl, parts, st);
+    }
+    return true;
+}
+
+template <typename T>
+static void launch_flux(const DevGeom& g, const DevState& s, const FlowParams& p, const TypeLists& tl,
+                        hipStream_t st, int parts, const LaunchShapes& ls) {
+    if (flux_small<T>(g, s, p, tl, st, parts)) return;
+    if (parts & 1) launch_class<0, T>(g, s, p, tl.fused_interior, tl.n_fused_interior, ls.flux_interior, st);
+    if (parts & 2) launch_class<1, T>(g, s, p, tl.fused_wall, tl.n_fused_wall, ls.flux_wall, st);
+}
+
 void launch_flux_fused(const DevGeom& g, const DevState& s, const FlowParams& p, const TypeLists& tl,
                        hipStream_t st, int parts, bool mixed, const LaunchShapes& ls) {
-    if (parts & 1) {
-        if (mixed)
-            launch_class<0, float>(g, s, p, tl.fused_interior, tl.n_fused_interior, ls.flux_interior, st);
-        else
-            launch_class<0, double>(g, s, p, tl.fused_interior, tl.n_fused_interior, ls.flux_interior, st);
-    }
-    if (parts & 2) {
-        if (mixed)
-            launch_class<1, float>(g, s, p, tl.fused_wall, tl.n_fused_wall, ls.flux_wall, st);
-        else
-            launch_class<1, double>(g, s, p, tl.fused_wall, tl.n_fused_wall, ls.flux_wall, st);
-    }
+    if (mixed) launch_flux<float>(g, s, p, tl, st, parts, ls);
+    else launch_flux<double>(g, s, p, tl, st, parts, ls);
 }
 
 }  // namespace mfcfd
