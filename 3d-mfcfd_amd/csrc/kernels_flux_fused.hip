@@ -19,15 +19,16 @@
 // A point is handled by a group of lanes, kFluxGroup = 4 of them unless the
 // points are few (flux_small), each taking every fourth neighbour, and the
 // group sums its partial residuals at the end, in an order that does not
-// depend on the number of lanes.  Per lane this is the same work as one lane per point, but a resident
-// wave holds 64 / kFluxGroup points instead of 64: the neighbour data of all
-// points in flight on one XCD then fits its 4 MB L2.  With one lane per point
+// depend on the number of lanes.  Per lane this is the same work as one lane
+// per point, but a resident wave holds 64 / kFluxGroup points instead of 64:
+// the neighbour data of all points in flight on one XCD then fits its 4 MB L2.  With one lane per point
 // at the 8 resident waves per CU the FP64 kernel's registers allow, each
 // point's q, qm and dq were fetched from HBM about 19 times per launch.
 #include <hip/hip_runtime.h>
 
 #include "device_common.h"
 #include "device_state.h"
+#include "erf_exp.h"
 #include "kernels.h"
 #include "qlskum_math.h"
 
@@ -39,26 +40,79 @@ namespace {
 
 constexpr int kFluxGroup = 4;
 
-// quantities of one reconstructed end state shared by every flux of the edge
+// quantities of one reconstructed end state shared by every flux of the edge;
+// b_scale: B = b_scale*exp(-S*S) (FP64), or sqrt(pi*beta) (FP32)
 template <typename T>
 struct EndState {
-    T rho, pr, ut[3], sqrt_beta, sqrt_pi_beta, e5;
+    T rho, pr, ut[3], sqrt_beta, b_scale, e5;
 };
 
 template <typename T>
-__device__ __forceinline__ EndState<T> end_state(const T prim[5], const Frame<T>& f, T pi) {
-    EndState<T> e;
-    const T u1 = prim[1], u2 = prim[2], u3 = prim[3];
-    e.rho = prim[0];
-    e.pr = prim[4];
+__device__ __forceinline__ void rotate_end(EndState<T>& e, const Frame<T>& f, T u1, T u2, T u3) {
     e.ut[0] = f.t1[0] * u1 + f.t1[1] * u2 + f.t1[2] * u3;
     e.ut[1] = f.t2[0] * u1 + f.t2[1] * u2 + f.t2[2] * u3;
     e.ut[2] = f.n[0] * u1 + f.n[1] * u2 + f.n[2] * u3;
-    const T beta = ddiv(T(0.5) * e.rho, e.pr);
-    e.sqrt_beta = dsqrt_fast(beta);
-    e.sqrt_pi_beta = dsqrt_fast(pi * beta);
     const T u_sqr = e.ut[0] * e.ut[0] + e.ut[1] * e.ut[1] + e.ut[2] * e.ut[2];
     e.e5 = T(2.5) * e.pr + T(0.5) * e.rho * u_sqr;
+}
+
+// The limited reconstruction at one end of an edge (limiters.f90:18-40), its
+// primitive variables (qvariables_to_primitive_variables.f90:16-30) and what
+// the fluxes take from them.
+__device__ __forceinline__ EndState<float> edge_end(const float q[5], const float* dq, const float* qm, float epsi2,
+                                                    float delx, float dely, float delz, const Frame<float>& f,
+                                                    float pi) {
+    float prim[5];
+    reconstruct_end<float>(q, dq, qm, epsi2, delx, dely, delz, prim);
+    EndState<float> e;
+    e.rho = prim[0];
+    e.pr = prim[4];
+    const float beta = ddiv(0.5f * e.rho, e.pr);
+    e.sqrt_beta = dsqrt_fast(beta);
+    e.b_scale = dsqrt_fast(pi * beta);
+    rotate_end(e, f, prim[1], prim[2], prim[3]);
+    return e;
+}
+
+// FP64: the same quantities with fewer divisions and roots.
+//   limiter   num/den with the common factor del_neg taken out of both;
+//   beta      is -q5/2 itself (the reference gets it back as 0.5*rho/p), and
+//             1/beta, sqrt(beta) and 1/sqrt(beta) come from one root;
+//   rho       exp(q1 + beta*u*u - 2.5*log(beta)) as exp(q1 + beta*u*u) *
+//             beta^(-5/2), with no logarithm.
+// Against the reference's expressions in 64-bit-mantissa arithmetic, over
+// states of Mach 0 to 3, the flux residual's error is that of the same
+// expressions in doubles or up to 1% less.
+__device__ __forceinline__ EndState<double> edge_end(const double q[5], const double* dq, const double* qm,
+                                                     double epsi2, double delx, double dely, double delz,
+                                                     const Frame<double>& f, double pi) {
+    double qt[5];
+#pragma unroll
+    for (int r = 0; r < 5; ++r) {
+        const double dn = -0.5 * (delx * dq[3 * r] + dely * dq[3 * r + 1] + delz * dq[3 * r + 2]);
+        const double dp = (dn > 0.0 ? qm[2 * r] : qm[2 * r + 1]) - q[r];
+        const double a = fma(dp, dp, epsi2), dn2 = 2.0 * dn;
+        const double ratio = div_refined(fma(dn2, dp, a), fma(dn, dn2 + dp, a));
+        // a NaN ratio or a NaN dn gives 1
+        const double phi = __builtin_fabs(dn) > kLimiterThreshold ? __builtin_fmin(ratio, 1.0) : 1.0;
+        qt[r] = fma(phi, dn, q[r]);
+    }
+    EndState<double> e;
+    const double beta = -0.5 * qt[4];
+    const RootOf y = root_of(beta);
+    // y^2 and y^5 with what their roundings drop (l2, l5) and the root's own
+    // correction y.e added at the end
+    const double y2 = y.y * y.y, l2 = fma(y.y, y.y, -y2);
+    const double temp = 0.5 * (y2 + fma(y2, y.e, l2));   // 0.5/beta
+    const double u1 = qt[1] * temp, u2 = qt[2] * temp, u3 = qt[3] * temp;
+    const double y4 = y2 * y2, y5 = y4 * y.y;
+    const double l4 = fma(2.0 * y2, l2, fma(y2, y2, -y4));
+    const double l5 = fma(y4, y.y, -y5) + fma(l4, y.y, 2.5 * y.e * y5);
+    e.rho = exp_series(fma(beta, fma(u3, u3, fma(u2, u2, u1 * u1)), qt[0])) * (y5 + l5);
+    e.pr = e.rho * temp;
+    e.sqrt_beta = sqrt_of(y);
+    e.b_scale = rsqrt_of(y, 0.28209479177387814);   // 0.5/sqrt(pi)
+    rotate_end(e, f, u1, u2, u3);
     return e;
 }
 
@@ -66,9 +120,15 @@ __device__ __forceinline__ EndState<T> end_state(const T prim[5], const Frame<T>
 template <int A, typename T>
 __device__ __forceinline__ void axis_terms(const EndState<T>& e, T& B, T& er) {
     const T S = e.ut[A] * e.sqrt_beta;
-    const T ex = dexp(-S * S);
-    B = ddiv(T(0.5) * ex, e.sqrt_pi_beta);
-    er = derf_e(S, ex);
+    T ex;
+    if constexpr (sizeof(T) == 8) {
+        erf_exp(S, er, ex);
+        B = e.b_scale * ex;
+    } else {
+        ex = dexp(-S * S);
+        B = ddiv(T(0.5) * ex, e.b_scale);
+        er = derf_e(S, ex);
+    }
 }
 
 // split_fluxes.f90 flux_G{x,y,z}{p,n}; sg = +1 or -1
@@ -253,17 +313,14 @@ __device__ __forceinline__ void flux_point(const DevGeom& g, const DevState& s, 
             const double delt = delx * f.t2[0] + dely * f.t2[1] + delz * f.t2[2];
             const double deln = delx * f.n[0] + dely * f.n[1] + delz * f.n[2];
             const double wgt = wls_weight<UW>(dels, delt, deln, fp.power);
-            T prim[5], qi[5];
+            T qi[5], qk[5];
 #pragma unroll
             for (int r = 0; r < 5; ++r) qi[r] = qip[r];
-            reconstruct_end<T>(qi, dqi, qmi, epsi2_i, T(delx), T(dely), T(delz), prim);
-            const EndState<T> ei = end_state(prim, ft, pi);
-            T qk[5];
+            const EndState<T> ei = edge_end(qi, dqi, qmi, epsi2_i, T(delx), T(dely), T(delz), ft, pi);
 #pragma unroll
             for (int r = 0; r < 5; ++r) qk[r] = qa.qp(k)[r];
-            reconstruct_end<T>(qk, qa.dqp(k), qa.qmp(k), T(limiter_epsi2(fp.vl_const, pk.w)), T(delx), T(dely),
-                               T(delz), prim);
-            const EndState<T> ek = end_state(prim, ft, pi);
+            const EndState<T> ek = edge_end(qk, qa.dqp(k), qa.qmp(k), T(limiter_epsi2(fp.vl_const, pk.w)), T(delx),
+                                            T(dely), T(delz), ft, pi);
             if (CLASS == 0) {
                 interior_axis<0>(ei, ek, bits, cf, wgt, dels, delt, deln, sum);
                 interior_axis<1>(ei, ek, bits, cf, wgt, dels, delt, deln, sum);
@@ -296,6 +353,7 @@ __device__ __forceinline__ void flux_point(const DevGeom& g, const DevState& s, 
 template <int CLASS, bool UW, typename T, int WAVES>
 __global__ void __launch_bounds__(kBlock, WAVES) k_flux_fused(DevGeom g, DevState s, FlowParams fp, const int* idx,
                                                              int count) {
+    if constexpr (sizeof(T) == 8) load_erf_nodes();
     const unsigned t = (unsigned)xcd_index();
     const int m = (int)(t / kFluxGroup);
     if (m >= count) return;  // whole groups: blocks hold a multiple of kFluxGroup lanes
@@ -311,10 +369,13 @@ __host__ __device__ inline int small_blocks(int points, int lanes) {
 // Both classes of a cloud that does not fill the chip in one launch, GG lanes
 // per point of the general class, whose points take longer and come first,
 // and GI per point of the interior one, from the next block on.
+// (FP64: two waves per SIMD; capped at three it spills 23 registers, and the
+// 250,000-point iteration takes 479 instead of 426 us.)
 template <bool UW, typename T, int GG, int GI>
-__global__ void __launch_bounds__(kBlock, GI == kFluxGroup ? 3 : 2)
+__global__ void __launch_bounds__(kBlock, sizeof(T) == 4 && GI == kFluxGroup ? 3 : 2)
     k_flux_small(DevGeom g, DevState s, FlowParams fp, const int* general, int n_general, const int* interior,
                  int n_interior) {
+    if constexpr (sizeof(T) == 8) load_erf_nodes();
     const int first = small_blocks(n_general, GG), b = (int)blockIdx.x;
     if (b < first) {
         const int t = xcd_block(b, first) * kBlock + (int)threadIdx.x, m = t / GG;
@@ -378,7 +439,8 @@ void launch_class(const DevGeom& g, const DevState& s, const FlowParams& p, cons
 // chip mostly idle by itself up to some 100,000 points, so it shares the
 // interior class's launch, until the interior class's registers (four waves
 // per SIMD in FP32 alone, three together) weigh more.  An iteration, in us,
-// before and after:
+// with four lanes and a launch per class, and so (both with the library's
+// functions in FP64):
 //     1,090 points, FP64   142 ->  41     mixed   97 ->  34   (32 + 32 lanes)
 //    20,000                176 ->  89            114 ->  56   (32 + 16)
 //    50,000                204 -> 143            133 ->  91   (16 + 4)

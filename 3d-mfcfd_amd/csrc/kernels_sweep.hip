@@ -373,7 +373,7 @@ __device__ __forceinline__ void finish_position(const SweepAsync& a, double* dU,
         w[2] = pack2(p32[4], 0.0f);
     } else {
         double pp[5];
-        conserved_to_prim(U, f, pp);
+        conserved_to_prim<double, true>(U, f, pp);
 #pragma unroll
         for (int r = 0; r < 5; ++r) w[r] = (unsigned long long)__double_as_longlong(pp[r]);
     }
@@ -451,7 +451,7 @@ __global__ void __launch_bounds__(kBlock) k_sweep_snap(DevGeom g, DevState s, co
         double U[5], prim[5];
 #pragma unroll
         for (int r = 0; r < 5; ++r) U[r] = dU[5 * (long long)k + r] + s.U[5 * (long long)k + r];
-        conserved_to_prim(U, load_frame(g.frame, k), prim);
+        conserved_to_prim<double, true>(U, load_frame(g.frame, k), prim);
 #pragma unroll
         for (int r = 0; r < 5; ++r) a.pold[5 * (long long)k + r] = prim[r];
     } else if (e < (long long)a.n_old + a.n_old_src) {

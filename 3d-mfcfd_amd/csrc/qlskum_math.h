@@ -1,13 +1,13 @@
 // qlskum_math.h -- per-point q-LSKUM arithmetic shared by the HIP kernels.
 //
 // Every routine keeps the reference's expression order (Fortran a+b+c is
-// (a+b)+c, a*b*c is (a*b)*c) and the FP64 kernels are compiled with
-// -ffp-contract=off, so the only differences from the reference CPU build
-// come from the device exp/log/erf (ocml vs glibc, within an ulp or two) --
-// and, in the sync-free sweeps, from the sweep form of the split fluxes
-// (SWEEP below: two roots from one reciprocal square root, within 2 ulp)
-// and from kernels_sweep.hip's -ffp-contract=on (a*b + c fused within an
-// expression, identically at every call site).
+// (a+b)+c, a*b*c is (a*b)*c) and kernels_fp64.hip is compiled with
+// -ffp-contract=off, so its only differences from the reference CPU build
+// come from the device exp/log/erf (ocml vs glibc, within an ulp or two).
+// The sync-free sweeps take the sweep form of the split fluxes (SWEEP below:
+// one refined quotient and root), the fused flux kernel its own forms
+// (kernels_flux_fused.hip), and both units -ffp-contract=on (a*b + c fused
+// within an expression, identically at every call site).
 // Routines are templated on the arithmetic type T so the mixed-precision
 // kernels reuse them with float, where division, square root and erf take
 // the faster forms defined below.
@@ -47,52 +47,84 @@ template <> __device__ __forceinline__ float dsqrt_fast<float>(float x) { return
 // In FP32 arithmetic the pair stays within 4e-7 of erf over all x; both
 // branches are evaluated and one selected, so lanes do not diverge.
 template <typename T> __device__ __forceinline__ T derf_e(T x, T ex);
-// FP64 erf is kept out of line: inlined, the library routine's working
-// registers add to everything live around it and take the fused flux kernel
-// from ~150 to ~223 VGPRs (2 instead of 3 resident waves per SIMD)
+// FP64 erf is kept out of line (list-by-list and level kernels): inlined, the
+// library routine's working registers add to everything live around it
 __device__ __attribute__((noinline)) inline double erf_out_of_line(double x) { return erf(x); }
 template <> __device__ __forceinline__ double derf_e<double>(double x, double) { return erf_out_of_line(x); }
-// SWEEP selects the sweep form of the split fluxes, for kernels whose flux
-// evaluations sit on a dependency chain.  In FP64 it
-//   * inlines the library erf (registers are spare there: 3% shorter), and
-//   * takes sqrt(beta) and 0.5/sqrt(pi*beta) from one reciprocal square root
-//     of beta (beta_roots), so that the coefficient B is one multiply after
-//     exp instead of an IEEE division (within 2 ulp of the IEEE forms).
-// FP32 is the same in both forms.
-template <typename T, bool SWEEP>
-__device__ __forceinline__ T derf_sel(T x, T ex) {
-    if constexpr (SWEEP && sizeof(T) == 8) return erf(x);
-    else return derf_e(x, ex);
+// a/b for normal b: the reciprocal estimate (v_rcp_f64, about 2^-23) refined by
+// one Newton step, and the quotient by its residual.  Half an ulp beyond
+// rounding, in 6 instructions instead of some 11.
+__device__ __forceinline__ double div_refined(double a, double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(r, fma(-b, r, 1.0), r);
+    const double q = a * r;
+    return fma(r, fma(-b, q, a), q);
 }
 
-// 1/sqrt(x) to double precision: the hardware estimate (v_rsq_f64) refined
-// by two Newton-Raphson steps y <- y*(1.5 - 0.5*x*y*y); x is a positive
-// normal number
-__device__ __forceinline__ double rsqrt_refined(double x) {
-    const double hx = 0.5 * x;
-    double y = __builtin_amdgcn_rsq(x);
-    y = y * fma(-hx, y * y, 1.5);
-    y = y * fma(-hx, y * y, 1.5);
-    return y;
+// y ~ 1/sqrt(x) and h = x*y, with e = 1 - x*y*y to double-double accuracy, so
+// that 1/sqrt(x) = y*(1 + e/2), sqrt(x) = h*(1 + e/2), 1/x = y*y*(1 + e), up
+// to e*e < 2^-80: every power of x wanted is one product and one correction
+// away.  The estimate (v_rsq_f64, about 2^-23) and one Newton step.
+struct RootOf {
+    double y, h, e;
+};
+__device__ __forceinline__ RootOf root_of(double x) {
+    RootOf o;
+    const double y0 = __builtin_amdgcn_rsq(x);
+    const double h0 = x * y0;
+    o.y = fma(0.5 * y0, fma(-h0, y0, 1.0), y0);
+    o.h = x * o.y;
+    o.e = fma(-fma(x, o.y, -o.h), o.y, fma(-o.h, o.y, 1.0));
+    return o;
+}
+__device__ __forceinline__ double sqrt_of(const RootOf& r) { return fma(0.5 * r.h, r.e, r.h); }
+// c/sqrt(x)
+__device__ __forceinline__ double rsqrt_of(const RootOf& r, double c) {
+    const double v = c * r.y;
+    return fma(0.5 * v, r.e, v);
 }
 
-// sb = sqrt(beta) and hb = 0.5/sqrt(pi*beta), so that B = exp(-S*S)*hb
+// The part of a split flux that depends on beta = 0.5*rho/p: sb = sqrt(beta),
+// and what half_range takes B from.  SWEEP selects the sweep form, for
+// kernels whose flux evaluations sit on a dependency chain: in FP64 one
+// refined quotient and one root instead of IEEE divisions and square roots
+// (1M FP64 sweep 9.0 -> 8.8 ms), and the library erf inlined: registers are
+// spare there.  (erf_exp.h has fewer instructions but no shorter chain of
+// them: 9.0 ms.)  FP32 is the same in both forms.
+template <typename T>
+struct BetaTerms {
+    T beta, sb, hb;   // hb: 0.5/sqrt(pi*beta), FP64 sweep form only
+};
 template <typename T, bool SWEEP>
-__device__ __forceinline__ void beta_roots(T beta, T pi, T& sb, T& hb) {
+__device__ __forceinline__ BetaTerms<T> beta_terms(T rho, T pr) {
+    BetaTerms<T> o;
     if constexpr (SWEEP && sizeof(T) == 8) {
-        const T y = rsqrt_refined(beta);
-        sb = beta * y;
-        hb = (T(0.5) * rsqrt_refined(pi)) * y;
+        o.beta = div_refined(0.5 * rho, pr);
+        const RootOf r = root_of(o.beta);
+        o.sb = sqrt_of(r);
+        o.hb = rsqrt_of(r, 0.28209479177387814);   // 0.5/sqrt(pi)
     } else {
-        sb = dsqrt_fast(beta);
-        hb = T(0);   // unused: the reference form divides by sqrt(pi*beta)
+        o.beta = ddiv(T(0.5) * rho, pr);
+        o.sb = dsqrt_fast(o.beta);
+        o.hb = T(0);
     }
+    return o;
 }
 
+// erf(S) and B = 0.5*exp(-S*S)/sqrt(pi*beta) of one component, S = u*sb
 template <typename T, bool SWEEP>
-__device__ __forceinline__ T b_coef(T ex, T hb, T pi, T beta) {
-    if constexpr (SWEEP && sizeof(T) == 8) return ex * hb;
-    else return ddiv(T(0.5) * ex, dsqrt_fast(pi * beta));
+__device__ __forceinline__ void half_range(T u, const BetaTerms<T>& bt, T pi, T& B, T& e) {
+    const T S = u * bt.sb;
+    T ex;
+    if constexpr (SWEEP && sizeof(T) == 8) {
+        ex = exp(-S * S);
+        e = erf(S);
+        B = ex * bt.hb;
+    } else {
+        ex = dexp(-S * S);
+        B = ddiv(T(0.5) * ex, dsqrt_fast(pi * bt.beta));
+        e = derf_e(S, ex);
+    }
 }
 template <> __device__ __forceinline__ float derf_e<float>(float x, float ex) {
     const float ax = x < 0.0f ? -x : x;
@@ -159,14 +191,10 @@ __device__ __forceinline__ void flux_half(int axis, int sign, const Frame<T>& f,
     const T ut1 = f.t1[0] * u1 + f.t1[1] * u2 + f.t1[2] * u3;
     const T ut2 = f.t2[0] * u1 + f.t2[1] * u2 + f.t2[2] * u3;
     const T un = f.n[0] * u1 + f.n[1] * u2 + f.n[2] * u3;
-    const T beta = ddiv(T(0.5) * rho, pr);
     const T ua = axis == 0 ? ut1 : (axis == 1 ? ut2 : un);
-    T sb, hb;
-    beta_roots<T, SWEEP>(beta, pi, sb, hb);
-    const T S = ua * sb;
-    const T ex = dexp(-S * S);
-    const T B = b_coef<T, SWEEP>(ex, hb, pi, beta);
-    const T e = derf_sel<T, SWEEP>(S, ex);
+    const BetaTerms<T> bt = beta_terms<T, SWEEP>(rho, pr);
+    T B, e;
+    half_range<T, SWEEP>(ua, bt, pi, B, e);
     const T A = T(0.5) * (sign > 0 ? T(1) + e : T(1) - e);
     const T Bs = sign > 0 ? B : -B;
     const T u_sqr = ut1 * ut1 + ut2 * ut2 + un * un;
@@ -190,18 +218,12 @@ __device__ __forceinline__ void flux_octant(int axis, int sign_a, int sign_n, co
     const T ut1 = f.t1[0] * u1 + f.t1[1] * u2 + f.t1[2] * u3;
     const T ut2 = f.t2[0] * u1 + f.t2[1] * u2 + f.t2[2] * u3;
     const T un = f.n[0] * u1 + f.n[1] * u2 + f.n[2] * u3;
-    const T beta = ddiv(T(0.5) * rho, pr);
     const T ua = axis == 0 ? ut1 : ut2;
-    T sb, hb;
-    beta_roots<T, SWEEP>(beta, pi, sb, hb);
-    const T Sa = ua * sb;
-    const T S3 = un * sb;
-    const T exa = dexp(-Sa * Sa), ex3 = dexp(-S3 * S3);
-    const T Ba = b_coef<T, SWEEP>(exa, hb, pi, beta);
-    const T B3 = b_coef<T, SWEEP>(ex3, hb, pi, beta);
-    const T ea = derf_sel<T, SWEEP>(Sa, exa);
+    const BetaTerms<T> bt = beta_terms<T, SWEEP>(rho, pr);
+    T Ba, ea, B3, e3;
+    half_range<T, SWEEP>(ua, bt, pi, Ba, ea);
+    half_range<T, SWEEP>(un, bt, pi, B3, e3);
     const T Aa = T(0.5) * (sign_a > 0 ? T(1) + ea : T(1) - ea);
-    const T e3 = derf_sel<T, SWEEP>(S3, ex3);
     const T A3 = T(0.5) * (sign_n > 0 ? T(1) + e3 : T(1) - e3);
     const T u_sqr = ut1 * ut1 + ut2 * ut2 + un * un;
     const T temp1 = (ua * Aa + (sign_a > 0 ? Ba : -Ba));
@@ -268,10 +290,13 @@ __device__ __forceinline__ void qtilde_to_primitive(const T q[5], T prim[5]) {
 
 // get_primitive_vector.f90:10-41 / conserved_to_primitive_vector.f90:10-42:
 // local-frame conserved vector of a point -> global primitive vector
-template <typename T>
+// (SWEEP: 1/rho as a refined quotient)
+template <typename T, bool SWEEP = false>
 __device__ __forceinline__ void conserved_to_prim(const T U[5], const Frame<T>& f, T prim[5]) {
     prim[0] = U[0];
-    T temp = T(1) / U[0];
+    T temp;
+    if constexpr (SWEEP && sizeof(T) == 8) temp = div_refined(1.0, U[0]);
+    else temp = T(1) / U[0];
     const T u2 = f.t1[0] * U[1] + f.t2[0] * U[2] + f.n[0] * U[3];
     const T u3 = f.t1[1] * U[1] + f.t2[1] * U[2] + f.n[1] * U[3];
     const T u4 = f.t1[2] * U[1] + f.t2[2] * U[2] + f.n[2] * U[3];
