@@ -1716,7 +1716,7 @@ int mfcfd_autotune(mfcfd_ctx* c, int repeats, mfcfd_tuning* out) {
                     best.qderiv = ks;
                 }
             }
-        for (int lds : caps(best.qderiv.block, {8, 12})) {
+        for (int lds : caps(best.qderiv.block, {8, 12, 16})) {
             KernelShape ks = best.qderiv;
             ks.lds = lds;
             double ms = 0.0;

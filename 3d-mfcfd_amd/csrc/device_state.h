@@ -77,14 +77,14 @@ struct DevState {
     double* qm;
     double* dq;
     double* delt;
-    double* tsden;   // [n] |u| + 3 sqrt(p/rho) of each point, the local time step's denominator
+    double* tsden;   // [n] 1/(|u| + 3 sqrt(p/rho))^2 of each point, the local time step is cfl*sqrt(min dist^2*tsden)
     double* flux_res;
     double* delUp;
     double* delUn;
     double* dinv;
     // mixed precision: q, qm, dq held in FP32 (the reference layouts, except
     // that q32 holds kQ32Stride floats per point: q, then the time step's
-    // denominator tsden in FP32, which the q-derivative kernel then reads
+    // weight tsden in FP32, which the q-derivative kernel then reads
     // with the same two loads as q)
     float* q32;
     float* qm32;

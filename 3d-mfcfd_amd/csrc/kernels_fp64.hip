@@ -115,6 +115,15 @@ __device__ __forceinline__ void conserved_point(const DevState& s, long long k, 
     for (int r = 0; r < 5; ++r) s.U[5 * k + r] = U[r];
 }
 
+// timestep_delt.f90:40-42: the neighbour-only part of the local step,
+// cfl*dist/(|u| + 3*sqrt(p/rho)), as 1/(...)^2: the step is then
+// cfl*sqrt(min(dist^2 * this)), one product per neighbour where a root and a
+// quotient per neighbour were a quarter of the q-derivative kernel's loop
+__device__ __forceinline__ double timestep_weight(double rho, double u1, double u2, double u3, double pr) {
+    const double den = __builtin_sqrt(u1 * u1 + u2 * u2 + u3 * u3) + 3.0 * __builtin_sqrt(pr / rho);
+    return 1.0 / (den * den);
+}
+
 template <typename QT>
 __device__ __forceinline__ void q_point(const DevState& s, long long k, const double p[5]) {
     const double rho = p[0], u1 = p[1], u2 = p[2], u3 = p[3], pr = p[4];
@@ -129,10 +138,9 @@ __device__ __forceinline__ void q_point(const DevState& s, long long k, const do
     QT* qo = qarrays<QT>(s).qp(k);
 #pragma unroll
     for (int r = 0; r < 5; ++r) qo[r] = QT(q[r]);
-    // timestep_delt.f90:40-42: the neighbour-only part of the local step
-    const double den = __builtin_sqrt(u1 * u1 + u2 * u2 + u3 * u3) + 3.0 * __builtin_sqrt(pr / rho);
-    s.tsden[k] = den;
-    if (sizeof(QT) == 4) qo[5] = QT(den);
+    const double w = timestep_weight(rho, u1, u2, u3, pr);
+    s.tsden[k] = w;
+    if (sizeof(QT) == 4) qo[5] = QT(w);
 }
 
 template <bool DO_U, bool DO_Q, typename QT>
@@ -146,13 +154,13 @@ __global__ void __launch_bounds__(kBlock) k_conserved_q(DevGeom g, DevState s) {
     if (DO_Q) q_point<QT>(s, k, p);
 }
 
-// the time step's denominators alone (time step called outside an iteration)
+// the time step's weights alone (time step called outside an iteration)
 __global__ void __launch_bounds__(kBlock) k_timestep_den(DevGeom g, DevState s) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= g.n) return;
     const double* p = s.prim + 5 * (long long)k;
     const double rho = p[0], u1 = p[1], u2 = p[2], u3 = p[3], pr = p[4];
-    s.tsden[k] = __builtin_sqrt(u1 * u1 + u2 * u2 + u3 * u3) + 3.0 * __builtin_sqrt(pr / rho);
+    s.tsden[k] = timestep_weight(rho, u1, u2, u3, pr);
 }
 
 // ---------------------------------------------------------------------------
@@ -166,8 +174,64 @@ __global__ void __launch_bounds__(kBlock) k_timestep_den(DevGeom g, DevState s) 
 // neighbour; the group combines its partial sums, maxima and minima at the
 // end.  Fewer points in flight per XCD keep their neighbours' q, prim and
 // positions resident in its L2.
+//
+// What bounds it: its neighbour loads (7 per neighbour in FP64, 5 in the mixed
+// form), then the arithmetic of the loop and of the solve.  Multiply-adds are
+// fused, the solve takes the six cofactors once for all 15 derivatives, and
+// the FP64 form is compiled for two waves per SIMD: its 166 registers fit
+// three, where a cap at four waves spilled 24 of them into the loop.  2M
+// cloud, FP64: 881 -> 629 us.
 constexpr int kQdGroup = 4;
-template <bool DO_DQ, bool DO_DT, bool UW, typename QT, int WAVES = 4>
+
+template <typename T>
+__device__ __forceinline__ T fma_of(T a, T b, T c) {
+    if constexpr (sizeof(T) == 8) return __builtin_fma(a, b, c);
+    else return __builtin_fmaf(a, b, c);
+}
+
+// one neighbour's part of the weighted normal matrix
+template <bool UW>
+__device__ __forceinline__ void add_geo(Geo6<double>& geo, double dx, double dy, double dz, double w) {
+    const double wx = UW ? dx : dx * w, wy = UW ? dy : dy * w, wz = UW ? dz : dz * w;
+    geo.xx = __builtin_fma(wx, dx, geo.xx);
+    geo.yy = __builtin_fma(wy, dy, geo.yy);
+    geo.zz = __builtin_fma(wz, dz, geo.zz);
+    geo.xy = __builtin_fma(wx, dy, geo.xy);
+    geo.yz = __builtin_fma(wy, dz, geo.yz);
+    geo.zx = __builtin_fma(wz, dx, geo.zx);
+}
+
+__device__ __forceinline__ void sum_geo(Geo6<double>& geo) {
+    geo.xx = group_sum<kQdGroup>(geo.xx);
+    geo.yy = group_sum<kQdGroup>(geo.yy);
+    geo.zz = group_sum<kQdGroup>(geo.zz);
+    geo.xy = group_sum<kQdGroup>(geo.xy);
+    geo.yz = group_sum<kQdGroup>(geo.yz);
+    geo.zx = group_sum<kQdGroup>(geo.zx);
+}
+
+// the inverse of the normal matrix (q_derivatives.f90:85-107 solves by
+// Cramer's rule, component by component)
+struct Inverse6 {
+    double xx, yy, zz, xy, yz, zx;
+    __device__ __forceinline__ explicit Inverse6(const Geo6<double>& g) {
+        const double f = 1.0 / cramer_det(g);
+        xx = (g.yy * g.zz - g.yz * g.yz) * f;
+        yy = (g.xx * g.zz - g.zx * g.zx) * f;
+        zz = (g.xx * g.yy - g.xy * g.xy) * f;
+        xy = (g.zx * g.yz - g.xy * g.zz) * f;
+        yz = (g.xy * g.zx - g.xx * g.yz) * f;
+        zx = (g.xy * g.yz - g.zx * g.yy) * f;
+    }
+    template <typename QT>
+    __device__ __forceinline__ void solve(double a, double b, double c, QT* out) const {
+        out[0] = QT(__builtin_fma(xx, a, __builtin_fma(xy, b, zx * c)));
+        out[1] = QT(__builtin_fma(xy, a, __builtin_fma(yy, b, yz * c)));
+        out[2] = QT(__builtin_fma(zx, a, __builtin_fma(yz, b, zz * c)));
+    }
+};
+
+template <bool DO_DQ, bool DO_DT, bool UW, typename QT, int WAVES = sizeof(QT) == 8 ? 2 : 4>
 __global__ void __launch_bounds__(kBlock, WAVES) k_qderiv_timestep(DevGeom g, DevState s, FlowParams fp) {
     const unsigned t = (unsigned)xcd_index();
     const int i = (int)(t / kQdGroup);
@@ -189,7 +253,7 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_qderiv_timestep(DevGeom g, De
             sx[r] = sy[r] = sz[r] = QT(0);
         }
     }
-    double min_delt = 1.0;
+    double min_step = __builtin_inf();   // of dist^2 * timestep_weight
     for (int j = lane; j < nb; j += kQdGroup) {
         const int k = cn[j];
         const double4 pk = g.pos[k];
@@ -206,37 +270,26 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_qderiv_timestep(DevGeom g, De
                 if (qk[r] < qmin[r]) qmin[r] = qk[r];
             }
             const double weights = wls_weight<UW>(delx, dely, delz, fp.power);
-            geo.xx = geo.xx + delx * delx * weights;
-            geo.yy = geo.yy + dely * dely * weights;
-            geo.zz = geo.zz + delz * delz * weights;
-            geo.xy = geo.xy + delx * dely * weights;
-            geo.yz = geo.yz + dely * delz * weights;
-            geo.zx = geo.zx + delz * delx * weights;
+            add_geo<UW>(geo, delx, dely, delz, weights);
             const QT wx = QT(weights * delx), wy = QT(weights * dely), wz = QT(weights * delz);
 #pragma unroll
             for (int r = 0; r < 5; ++r) {
                 const QT t = qk[r] - qi[r];
-                sx[r] = sx[r] + wx * t;
-                sy[r] = sy[r] + wy * t;
-                sz[r] = sz[r] + wz * t;
+                sx[r] = fma_of(wx, t, sx[r]);
+                sy[r] = fma_of(wy, t, sy[r]);
+                sz[r] = fma_of(wz, t, sz[r]);
             }
         }
         if (DO_DT) {
-            // timestep_delt.f90:34-47, the neighbour's denominator read, not recomputed
-            const double dist = __builtin_sqrt(delx * delx + dely * dely + delz * delz);
+            // timestep_delt.f90:34-47 (timestep_weight)
+            const double d2 = __builtin_fma(delx, delx, __builtin_fma(dely, dely, delz * delz));
             // the mixed form reads its FP32 copy, next to q
-            const double den = sizeof(QT) == 4 && DO_DQ ? (double)qa.qp(k)[5] : s.tsden[k];
-            const double delt = fp.cfl * dist / den;
-            if (delt < min_delt) min_delt = delt;
+            const double w = sizeof(QT) == 4 && DO_DQ ? (double)qa.qp(k)[5] : s.tsden[k];
+            min_step = __builtin_fmin(min_step, d2 * w);   // NaN never replaces a value
         }
     }
     if (DO_DQ) {
-        geo.xx = group_sum<kQdGroup>(geo.xx);
-        geo.yy = group_sum<kQdGroup>(geo.yy);
-        geo.zz = group_sum<kQdGroup>(geo.zz);
-        geo.xy = group_sum<kQdGroup>(geo.xy);
-        geo.yz = group_sum<kQdGroup>(geo.yz);
-        geo.zx = group_sum<kQdGroup>(geo.zx);
+        sum_geo(geo);
 #pragma unroll
         for (int r = 0; r < 5; ++r) {
             sx[r] = group_sum<kQdGroup>(sx[r]);
@@ -246,67 +299,65 @@ __global__ void __launch_bounds__(kBlock, WAVES) k_qderiv_timestep(DevGeom g, De
             qmin[r] = group_min<kQdGroup>(qmin[r]);
         }
     }
-    if (DO_DT) min_delt = group_min<kQdGroup>(min_delt);
+    if (DO_DT) min_step = group_min<kQdGroup>(min_step);
     if (lane != 0) return;
     if (DO_DQ) {
-        const double det = cramer_det(geo);
-        const double one_by_det = 1.0 / det;
+        const Inverse6 inv(geo);
 #pragma unroll
         for (int r = 0; r < 5; ++r) {
             qa.qmp(i)[r * 2 + 0] = qmax[r];
             qa.qmp(i)[r * 2 + 1] = qmin[r];
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-                qa.dqp(i)[r * 3 + c] =
-                    QT(cramer_num(geo, c, (double)sx[r], (double)sy[r], (double)sz[r]) * one_by_det);
+            inv.solve((double)sx[r], (double)sy[r], (double)sz[r], qa.dqp(i) + 3 * r);
         }
     }
-    if (DO_DT) s.delt[i] = min_delt;
+    if (DO_DT) s.delt[i] = __builtin_fmin(1.0, fp.cfl * __builtin_sqrt(min_step));
 }
 
 // q_derivatives.f90:116-201: inner iterations (second-order q-derivatives)
+// (kQdGroup lanes per point, as the first pass)
 template <bool UW>
-__global__ void __launch_bounds__(kBlock) k_qderiv_inner(DevGeom g, DevState s, FlowParams fp,
-                                                         double* temp) {
-    const int i = xcd_index();
-    if (i >= g.n) return;
+__global__ void __launch_bounds__(kBlock, 2) k_qderiv_inner(DevGeom g, DevState s, FlowParams fp, double* temp) {
+    const unsigned t = (unsigned)xcd_index();
+    const int i = (int)(t / kQdGroup);
+    const int lane = (int)(t % kQdGroup);
+    if (i >= g.n) return;  // whole groups
     const double4 pi4 = g.pos[i];
     const int nb = g.nbhs[i];
     const int* cn = g.conn + kConnCols * (long long)i;
+    const double *qi = s.q + 5 * (long long)i, *dqi = s.dq + 15 * (long long)i;
     double sx[5] = {0, 0, 0, 0, 0}, sy[5] = {0, 0, 0, 0, 0}, sz[5] = {0, 0, 0, 0, 0};
     Geo6<double> geo = {0, 0, 0, 0, 0, 0};
-    for (int j = 0; j < nb; ++j) {
+    for (int j = lane; j < nb; j += kQdGroup) {
         const int k = cn[j];
         const double4 pk = g.pos[k];
         const double delx = pk.x - pi4.x;
         const double dely = pk.y - pi4.y;
         const double delz = pk.z - pi4.z;
         const double weights = wls_weight<UW>(delx, dely, delz, fp.power);
-        geo.xx = geo.xx + delx * delx * weights;
-        geo.yy = geo.yy + dely * dely * weights;
-        geo.zz = geo.zz + delz * delz * weights;
-        geo.xy = geo.xy + delx * dely * weights;
-        geo.yz = geo.yz + dely * delz * weights;
-        geo.zx = geo.zx + delz * delx * weights;
+        add_geo<UW>(geo, delx, dely, delz, weights);
+        const double wx = weights * delx, wy = weights * dely, wz = weights * delz;
+        const double *qk = s.q + 5 * (long long)k, *dqk = s.dq + 15 * (long long)k;
 #pragma unroll
         for (int r = 0; r < 5; ++r) {
-            const double* dqi = s.dq + (5 * (long long)i + r) * 3;
-            const double* dqk = s.dq + (5 * (long long)k + r) * 3;
-            const double qti = s.q[5 * (long long)i + r] - 0.5 * (delx * dqi[0] + dely * dqi[1] + delz * dqi[2]);
-            const double qtn = s.q[5 * (long long)k + r] - 0.5 * (delx * dqk[0] + dely * dqk[1] + delz * dqk[2]);
-            const double t = qtn - qti;
-            sx[r] = sx[r] + weights * delx * t;
-            sy[r] = sy[r] + weights * dely * t;
-            sz[r] = sz[r] + weights * delz * t;
+            const double qti = qi[r] - 0.5 * (delx * dqi[3 * r] + dely * dqi[3 * r + 1] + delz * dqi[3 * r + 2]);
+            const double qtn = qk[r] - 0.5 * (delx * dqk[3 * r] + dely * dqk[3 * r + 1] + delz * dqk[3 * r + 2]);
+            const double d = qtn - qti;
+            sx[r] = __builtin_fma(wx, d, sx[r]);
+            sy[r] = __builtin_fma(wy, d, sy[r]);
+            sz[r] = __builtin_fma(wz, d, sz[r]);
         }
     }
-    const double det = cramer_det(geo);
-    const double one_by_det = 1.0 / det;
+    sum_geo(geo);
 #pragma unroll
-    for (int r = 0; r < 5; ++r)
+    for (int r = 0; r < 5; ++r) {
+        sx[r] = group_sum<kQdGroup>(sx[r]);
+        sy[r] = group_sum<kQdGroup>(sy[r]);
+        sz[r] = group_sum<kQdGroup>(sz[r]);
+    }
+    if (lane != 0) return;
+    const Inverse6 inv(geo);
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
-            temp[(5 * (long long)i + r) * 3 + c] = cramer_num(geo, c, sx[r], sy[r], sz[r]) * one_by_det;
+    for (int r = 0; r < 5; ++r) inv.solve(sx[r], sy[r], sz[r], temp + 15 * (long long)i + 3 * r);
 }
 
 // m values per point between an FP64 array of m per point and an FP32 array
@@ -1099,11 +1150,9 @@ void launch_q_derivatives(const DevGeom& g, const DevState& s, const FlowParams&
         hipLaunchKernelGGL((k_qderiv_timestep<true, false, false, double>), grid, dim3(kBlock), 0, st, g, s, p);
     for (int it = 0; it < p.inner_iterations; ++it) {
         if (p.power == 0.0)
-            hipLaunchKernelGGL(k_qderiv_inner<true>, dim3(grid_for(g.n, kBlock)), dim3(kBlock), 0, st, g, s, p,
-                               temp);
+            hipLaunchKernelGGL(k_qderiv_inner<true>, grid, dim3(kBlock), 0, st, g, s, p, temp);
         else
-            hipLaunchKernelGGL(k_qderiv_inner<false>, dim3(grid_for(g.n, kBlock)), dim3(kBlock), 0, st, g, s, p,
-                               temp);
+            hipLaunchKernelGGL(k_qderiv_inner<false>, grid, dim3(kBlock), 0, st, g, s, p, temp);
         hipLaunchKernelGGL(k_copy, dim3(grid_for(15LL * g.n, kBlock)), dim3(kBlock), 0, st, s.dq,
                            (const double*)temp, 15LL * g.n);
     }
@@ -1120,15 +1169,26 @@ void launch_qdt(const DevGeom& g, const DevState& s, const FlowParams& p, hipStr
     int block = ks.block > 0 && ks.block <= kBlock ? ks.block : kBlock;
     block -= block % kQdGroup;
     const dim3 grid(grid_for((long long)g.n * kQdGroup, block)), blk(block);
+    // The mixed form's 81 registers would let six waves share a SIMD; the points
+    // they hold overflow their XCD's L2.  Unless a shape was chosen, 40 KB of
+    // LDS per workgroup keep it to four (2M cloud 474 -> 442 us, 600,000 points
+    // 136 -> 128; the FP64 form's three waves: no difference).
+    const int lds = ks.block > 0 ? ks.lds : sizeof(QT) == 4 ? 40 * 1024 : 0;
     if (p.power != 0.0) {
-        hipLaunchKernelGGL((k_qderiv_timestep<true, true, false, QT>), grid, blk, ks.lds, st, g, s, p);
+        hipLaunchKernelGGL((k_qderiv_timestep<true, true, false, QT>), grid, blk, lds, st, g, s, p);
         return;
     }
-    switch (ks.waves) {
-        case 2: hipLaunchKernelGGL((k_qderiv_timestep<true, true, true, QT, 2>), grid, blk, ks.lds, st, g, s, p); break;
-        case 6: hipLaunchKernelGGL((k_qderiv_timestep<true, true, true, QT, 6>), grid, blk, ks.lds, st, g, s, p); break;
-        default: hipLaunchKernelGGL((k_qderiv_timestep<true, true, true, QT, 4>), grid, blk, ks.lds, st, g, s, p); break;
+    // the FP64 form has one variant: caps at four and six waves spill
+    if constexpr (sizeof(QT) == 4) {
+        if (ks.waves == 2 || ks.waves == 6) {
+            if (ks.waves == 2)
+                hipLaunchKernelGGL((k_qderiv_timestep<true, true, true, QT, 2>), grid, blk, lds, st, g, s, p);
+            else
+                hipLaunchKernelGGL((k_qderiv_timestep<true, true, true, QT, 6>), grid, blk, lds, st, g, s, p);
+            return;
+        }
     }
+    hipLaunchKernelGGL((k_qderiv_timestep<true, true, true, QT>), grid, blk, lds, st, g, s, p);
 }
 void launch_qderiv_timestep(const DevGeom& g, const DevState& s, const FlowParams& p, hipStream_t st,
                             const KernelShape& ks) {
