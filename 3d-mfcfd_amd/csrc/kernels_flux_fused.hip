@@ -403,27 +403,30 @@ void launch_class(const DevGeom& g, const DevState& s, const FlowParams& p, cons
     int block = ks.block > 0 && ks.block <= kBlock ? ks.block : kBlock;
     block -= block % kFluxGroup;
     const dim3 grid(grid_for((long long)count * kFluxGroup, block)), blk(block);
+    // the reservation counts the FP64 kernels' own table
+    constexpr int own = sizeof(T) == 8 ? kErfNodes * (int)sizeof(double2) : 0;
+    const int lds = ks.lds > own ? ks.lds - own : 0;
     if (p.power != 0.0) {
-        hipLaunchKernelGGL((k_flux_fused<CLASS, false, T, 2>), grid, blk, ks.lds, st, g, s, p, idx, count);
+        hipLaunchKernelGGL((k_flux_fused<CLASS, false, T, 2>), grid, blk, lds, st, g, s, p, idx, count);
         return;
     }
     switch (ks.waves) {
-        case 1: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 1>), grid, blk, ks.lds, st, g, s, p, idx, count); break;
-        case 3: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 3>), grid, blk, ks.lds, st, g, s, p, idx, count); break;
-        case 4: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 4>), grid, blk, ks.lds, st, g, s, p, idx, count); break;
+        case 1: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 1>), grid, blk, lds, st, g, s, p, idx, count); break;
+        case 3: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 3>), grid, blk, lds, st, g, s, p, idx, count); break;
+        case 4: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 4>), grid, blk, lds, st, g, s, p, idx, count); break;
         case 5:
             if constexpr (sizeof(T) == 4) {
-                hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 5>), grid, blk, ks.lds, st, g, s, p, idx, count);
+                hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 5>), grid, blk, lds, st, g, s, p, idx, count);
                 break;
             }
             [[fallthrough]];
         case 6:
             if constexpr (sizeof(T) == 4) {
-                hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 6>), grid, blk, ks.lds, st, g, s, p, idx, count);
+                hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 6>), grid, blk, lds, st, g, s, p, idx, count);
                 break;
             }
             [[fallthrough]];
-        default: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 2>), grid, blk, ks.lds, st, g, s, p, idx, count); break;
+        default: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 2>), grid, blk, lds, st, g, s, p, idx, count); break;
     }
 }
 

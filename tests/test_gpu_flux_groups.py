@@ -55,3 +55,22 @@ def test_sums_do_not_depend_on_the_lanes(precision, power, fillers):
     assert np.array_equal(got[0], s.download("prim"))
     assert np.array_equal(got[1], s.download("flux_res"))
     s.close()
+
+
+def test_autotuned_class_launches_fit_the_lds():
+    """Above the joint launch's sizes the autotuner reserves up to a CU's whole
+    LDS for a workgroup of the class kernels; the FP64 ones hold a table there."""
+    cl = shells(560000)
+    prim = np.tile(pc.freestream_prim(0.6, 2.0), (cl.n, 1))
+    print(f"[gpu] autotune, {cl.n} points", flush=True)
+    s = solver.Solver(cl, 0.6, 2.0, 0.2)
+    s.upload("prim", prim)
+    s.run(1, 2)
+    want = s.download("prim")
+    t = s.autotune(1)
+    for lds in (t["flux_interior_lds"], 163840):
+        s.set_tuning({**t, "flux_interior_lds": lds, "flux_wall_lds": lds})
+        s.upload("prim", prim)
+        s.run(1, 2)
+        assert np.array_equal(s.download("prim"), want)
+    s.close()
