@@ -156,7 +156,8 @@ struct mfcfd_ctx {
     int n_partial = 0;
     DevBuf<ResidualRecord> rec;
     DevBuf<double> hist;
-    ResidualRecord* host_rec = nullptr;  // pinned
+    ResidualRecord* host_rec = nullptr;      // pinned, and its address on the device
+    ResidualRecord* host_rec_dev = nullptr;
     // LU-SGS sweep plan of one sweep direction on the device (SweepPlan):
     // execution order, taken entries and their weights, snapshot and mark lists
     struct DevSweepDir {
@@ -639,23 +640,27 @@ int prepare_plan(mfcfd_ctx* c) {
     return build_plan(c, c->params.mode);
 }
 
+// to_host: the residual record goes to the pinned host copy as well, so that
+// fetch_record only has to wait
 int do_state_update(mfcfd_ctx* c, double* hist, int hist_index, const InstanceResidual* ir = nullptr,
-                    bool with_explicit_sweep = false) {
+                    bool with_explicit_sweep = false, bool to_host = false) {
     launch_state_update(c->geom(), c->state(), c->fp, c->tl, c->partial.p, c->partial_pos.p, c->n_partial,
-                        c->rec.p, hist, hist_index, c->stream, ir, with_explicit_sweep);
+                        c->rec.p, hist, hist_index, c->stream, ir, with_explicit_sweep,
+                        to_host ? c->host_rec_dev : nullptr);
     return launch_error("state update");
 }
 
 // the sweeps and the state update of one iteration; the explicit form's
 // sweep runs inside the state update's pass
-int do_sweeps_and_update(mfcfd_ctx* c, double* hist, int hist_index, const InstanceResidual* ir = nullptr) {
-    if (c->params.mode == MFCFD_EXPLICIT) return do_state_update(c, hist, hist_index, ir, true);
+int do_sweeps_and_update(mfcfd_ctx* c, double* hist, int hist_index, const InstanceResidual* ir, bool to_host) {
+    if (c->params.mode == MFCFD_EXPLICIT) return do_state_update(c, hist, hist_index, ir, true, to_host);
     int rc = do_sweeps(c);
     if (rc) return rc;
-    return do_state_update(c, hist, hist_index, ir);
+    return do_state_update(c, hist, hist_index, ir, false, to_host);
 }
 
-int do_iteration(mfcfd_ctx* c, double* hist, int hist_index, const InstanceResidual* ir = nullptr) {
+int do_iteration(mfcfd_ctx* c, double* hist, int hist_index, const InstanceResidual* ir = nullptr,
+                 bool to_host = false) {
     const DevGeom g = c->geom();
     const DevState s = c->state();
     launch_conserved_and_q(g, s, c->fp, c->stream);
@@ -668,7 +673,7 @@ int do_iteration(mfcfd_ctx* c, double* hist, int hist_index, const InstanceResid
     flux(c, kFluxAll);
     int rc = launch_error("iteration");
     if (rc) return rc;
-    return do_sweeps_and_update(c, hist, hist_index, ir);
+    return do_sweeps_and_update(c, hist, hist_index, ir, to_host);
 }
 
 // fpi_solver.f90:38-43
@@ -683,8 +688,11 @@ void residue_bookkeeping(mfcfd_ctx* c, int t, double res_new) {
     c->last_t = t;
 }
 
-int fetch_record(mfcfd_ctx* c) {
-    HIP_TRY(hipMemcpyAsync(c->host_rec, c->rec.p, sizeof(ResidualRecord), hipMemcpyDeviceToHost, c->stream));
+// the record of the last state update; on_host: that update wrote it to the
+// host copy itself (to_host)
+int fetch_record(mfcfd_ctx* c, bool on_host = false) {
+    if (!on_host)
+        HIP_TRY(hipMemcpyAsync(c->host_rec, c->rec.p, sizeof(ResidualRecord), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     collect_kernel_times(c);
     c->res_new = c->host_rec->res_new;
@@ -771,7 +779,8 @@ int mfcfd_create(int device, mfcfd_ctx** out) {
         return fail(MFCFD_EHIP, "hipStreamCreate failed");
     }
     if (c->rec.alloc(1) != hipSuccess ||
-        hipHostMalloc((void**)&c->host_rec, sizeof(ResidualRecord), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&c->host_rec, sizeof(ResidualRecord), hipHostMallocDefault) != hipSuccess ||
+        hipHostGetDevicePointer((void**)&c->host_rec_dev, c->host_rec, 0) != hipSuccess) {
         delete c;
         return fail(MFCFD_ENOMEM, "residual buffers");
     }
@@ -1480,16 +1489,16 @@ int mfcfd_implicit_forward_backward_sweeps(mfcfd_ctx* c) {
 int mfcfd_state_update(mfcfd_ctx* c) {
     int rc = check_ctx(c, true);
     if (rc) return rc;
-    if ((rc = do_state_update(c, nullptr, 0))) return rc;
-    return fetch_record(c);
+    if ((rc = do_state_update(c, nullptr, 0, nullptr, false, true))) return rc;
+    return fetch_record(c, true);
 }
 
 int mfcfd_fpi_solver(mfcfd_ctx* c, int t, double* res_new, double* residue) {
     int rc = check_ctx(c, true);
     if (rc) return rc;
     if ((rc = prepare_plan(c))) return rc;
-    if ((rc = do_iteration(c, nullptr, 0))) return rc;
-    if ((rc = fetch_record(c))) return rc;
+    if ((rc = do_iteration(c, nullptr, 0, nullptr, true))) return rc;
+    if ((rc = fetch_record(c, true))) return rc;
     residue_bookkeeping(c, t, c->res_new);
     if (res_new) *res_new = c->res_new;
     if (residue) *residue = c->residue;

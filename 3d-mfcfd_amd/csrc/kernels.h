@@ -160,12 +160,14 @@ struct InstanceResidual {
     double* chunk_sum;      // [n_chunks] scratch
 };
 // hist[hist_index] (or hist[*ir->counter] when ir is given) receives res_new;
+// host: null, or pinned host memory that receives *rec too
 // with_explicit_sweep: do the explicit form's sweep (launch_explicit_sweep)
 // in the same pass
 void launch_state_update(const DevGeom& g, const DevState& s, const FlowParams& p,
                          const TypeLists& tl, double* partial, int* partial_pos, int n_partial,
                          ResidualRecord* rec, double* hist, int hist_index, hipStream_t st,
-                         const InstanceResidual* ir = nullptr, bool with_explicit_sweep = false);
+                         const InstanceResidual* ir = nullptr, bool with_explicit_sweep = false,
+                         ResidualRecord* host = nullptr);
 int state_update_blocks(int n);
 
 }  // namespace mfcfd
