@@ -979,20 +979,28 @@ __global__ void k_supersonic(DevGeom g, DevState s, const int* out_idx, int n_ou
 
 // The partials' sum and maximum, in a fixed assignment to threads and a fixed
 // order: a wave's partials by butterfly, then the waves'.  One workgroup whose
-// latency every iteration pays: four waves and one barrier (a tree over 1024
-// threads' values in LDS, with ten, took 3 us more at 1,090 points).
+// latency every iteration pays: one barrier (a tree over 1024 threads' values
+// in LDS, with ten, took 3 us more at 1,090 points), a wave per 64 partials up
+// to sixteen (residual_threads; four waves took 16 us at 2M points and 66 at
+// 8M, sixteen 8 and 22), and four partials' loads in flight per thread.
 // host: null, or the pinned host copy of *rec
-__global__ void __launch_bounds__(kBlock) k_residual_final(const double* partial, const int* partial_pos,
-                                                           const int* partial_pt, const double* partial_max,
-                                                           int n_partial, int n_points,
-                                                           ResidualRecord* rec, double* hist, int hist_index,
-                                                           int* hist_counter, ResidualRecord* host) {
-    constexpr int kWaves = kBlock / 64;
+constexpr int kResidualBlock = 1024;
+int residual_threads(int n_partial) {
+    const int n = (n_partial + 63) / 64 * 64;
+    return n < kResidualBlock ? n : kResidualBlock;
+}
+__global__ void __launch_bounds__(kResidualBlock) k_residual_final(const double* partial, const int* partial_pos,
+                                                                   const int* partial_pt, const double* partial_max,
+                                                                   int n_partial, int n_points,
+                                                                   ResidualRecord* rec, double* hist, int hist_index,
+                                                                   int* hist_counter, ResidualRecord* host) {
+    constexpr int kWaves = kResidualBlock / 64;
     __shared__ double ssum[kWaves];
     __shared__ MaxPair smax[kWaves];
     double sum = 0.0;
     MaxPair mp = {0.0, 0x7fffffff, 0};
-    for (int b = threadIdx.x; b < n_partial; b += kBlock) {
+#pragma unroll 4
+    for (int b = threadIdx.x; b < n_partial; b += kResidualBlock) {
         sum = sum + partial[b];
         mp = max_pair(mp, MaxPair{partial_max[b], partial_pos[b], partial_pt[b]});
     }
@@ -1001,17 +1009,22 @@ __global__ void __launch_bounds__(kBlock) k_residual_final(const double* partial
         sum = sum + __shfl_xor(sum, o, 64);
         mp = max_pair(mp, MaxPair{__shfl_xor(mp.v, o, 64), __shfl_xor(mp.pos, o, 64), __shfl_xor(mp.point, o, 64)});
     }
-    if ((threadIdx.x & 63) == 0) {
+    const int lane = threadIdx.x & 63;
+    const int waves = blockDim.x >> 6;
+    if (lane == 0) {
         ssum[threadIdx.x >> 6] = sum;
         smax[threadIdx.x >> 6] = mp;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x >= 64) return;
+    sum = lane < waves ? ssum[lane] : 0.0;
+    mp = lane < waves ? smax[lane] : MaxPair{0.0, 0x7fffffff, 0};
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) {
-            sum = sum + ssum[w];
-            mp = max_pair(mp, smax[w]);
-        }
+    for (int o = kWaves / 2; o >= 1; o >>= 1) {
+        sum = sum + __shfl_xor(sum, o, 64);
+        mp = max_pair(mp, MaxPair{__shfl_xor(mp.v, o, 64), __shfl_xor(mp.pos, o, 64), __shfl_xor(mp.point, o, 64)});
+    }
+    if (threadIdx.x == 0) {
         ResidualRecord r;
         r.sum_res_sqr = sum;
         r.res_new = __builtin_sqrt(sum) / n_points;
@@ -1300,7 +1313,7 @@ void launch_state_update(const DevGeom& g, const DevState& s, const FlowParams& 
     if (backup)
         hipLaunchKernelGGL(k_copy, dim3(grid_for(5LL * g.n, kBlock)), dim3(kBlock), 0, st, s.delUp,
                            (const double*)s.delUn, 5LL * g.n);
-    hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(kBlock), 0, st, (const double*)partial,
+    hipLaunchKernelGGL(k_residual_final, dim3(1), dim3(residual_threads(n_partial)), 0, st, (const double*)partial,
                        (const int*)partial_pos, (const int*)partial_pt, (const double*)partial_max, n_partial,
                        g.n, rec, hist, hist_index, ir ? ir->counter : nullptr, host);
     if (ir) {

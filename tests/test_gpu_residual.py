@@ -13,7 +13,7 @@ solver = PKG.solver
 pc = PKG.pointcloud
 
 
-@pytest.mark.parametrize("partials,extra", [(32, 0), (64, 0), (64, 1), (256, 0), (256, 1)])
+@pytest.mark.parametrize("partials,extra", [(32, 0), (64, 0), (64, 1), (1024, 0), (1024, 1)])
 def test_residual_over_workgroups(partials, extra):
     n = 256 * partials + extra
     cl = pc.ellipsoid_cloud(n * 8 // 100, n * 4 // 100, n - n * 8 // 100 - n * 4 // 100, k=25, seed=9,
@@ -27,8 +27,8 @@ def test_residual_over_workgroups(partials, extra):
         rho = s.download("prim")[:, 0]
         res_new, _ = s.fpi_solver(t)
         # a term is two roundings of the densities on both sides, in the same
-        # order; a sum's error is at most its longest chain of additions (two
-        # butterflies of 6, twice 3 waves, 2 strides: under 24) half-ulps
+        # order; a sum's error is at most its longest chain of additions
+        # (butterflies of 6, 6 and 4, 3 waves, 2 strides: under 24) half-ulps
         term = np.where(cl.status < 2, (s.download("prim")[:, 0] - rho) ** 2, 0.0)
         total = math.fsum(term)
         rec = s.residual()
