@@ -92,8 +92,8 @@ typedef struct mfcfd_params {
 /* schedule of the implicit LU-SGS sweeps; both visit each point's
  * dependencies (stencil neighbours earlier in the sweep's alias order,
  * implicit_forward_and_reverse_sweeps.f90:26-85) before the point itself:
- *  ASYNC   one persistent launch per sweep; workgroups take points in sweep
- *          order and wait on per-point completion flags;
+ *  ASYNC   one persistent launch per sweep; workgroups take groups of points in
+ *          sweep order and wait on per-point published values;
  *  LEVELS  one launch per dependency level (host-built level sets). */
 #define MFCFD_SWEEP_ASYNC 0
 #define MFCFD_SWEEP_LEVELS 1
@@ -226,7 +226,8 @@ int mfcfd_run_graph(mfcfd_ctx *ctx, int t0, int n_iters, double *res_new_hist, d
 /* launch-shape autotuner (no counterpart in the reference).  Times, on the
  * bound cloud(s) and the current state, every compiled variant of the
  * gather kernels -- block size 64/128/256 x minimum waves per SIMD (the
- * register cap: 2/4/6 for the q-derivative kernel, 1..4 for the fused flux
+ * register cap: 2/4/6 for the mixed q-derivative kernel, whose FP64 form has one
+ * variant, 1..4 for the fused flux
  * kernels, 1..6 for their mixed-precision FP32 variants), then for the chosen shape an LDS reservation that caps the
  * resident waves per CU (fewer points in flight per XCD keep their
  * neighbours in that XCD's L2) -- and, in implicit mode, the sync-free
