@@ -598,12 +598,12 @@ int build_plan(mfcfd_ctx* c, int form) {
     };
     if ((rc = put(c->sw_fwd, plan.fwd))) return rc;
     if ((rc = put(c->sw_bwd, plan.bwd))) return rc;
-    if (c->pub.n == 0 && c->pub.alloc_fine(8ULL * n) != hipSuccess)
+    if (c->pub.n == 0 && c->pub.alloc_fine((size_t)kRecord<double> * n) != hipSuccess)
         return fail(MFCFD_ENOMEM, "sweep values (fine-grained)");
     // copy sources read as this sweep's delU: a slot each in dsrc
     const size_t n_src = std::max(plan.fwd.wait_src.size(), plan.bwd.wait_src.size());
     if (n_src > 0) {
-        if (c->dsrc.n < 5 * n_src && c->dsrc.alloc_fine(5 * n_src) != hipSuccess)
+        if (c->dsrc.n < kRecord<double> * n_src && c->dsrc.alloc_fine(kRecord<double> * n_src) != hipSuccess)
             return fail(MFCFD_ENOMEM, "sweep values (fine-grained)");
         for (int dir = 0; dir < 2; ++dir) {
             const std::vector<int>& ws = dir == 0 ? plan.fwd.wait_src : plan.bwd.wait_src;

@@ -75,11 +75,11 @@ struct SweepAsync {
     int n_old_src;
     const int* wait_src;        // copy sources read as this sweep's delU (slot j of dsrc: wait_src[j])
     int n_wait_src;
-    double* pub;                // [5n] published prim(U + delU) of the positions (completion marks;
+    double* pub;                // [kRecord n] published prim(U + delU) of the points (completion marks;
                                 // fine-grained memory)
     double* pold;               // [5n] prim(U + delU) before the sweep, for old entries
     double* dold;               // [5n] delU before the sweep, for copies from old sources (may be null)
-    double* dsrc;               // [5 n_wait_src] published delU of the copy sources read as this
+    double* dsrc;               // [kRecord n_wait_src] published delU of the copy sources read as this
                                 // sweep's value (fine-grained; may be null)
     const int* src_slot;        // [n] slot of each point in dsrc, -1 if none (may be null)
     unsigned* ctr;              // [kSweepCounters] ticket counter, finished workgroups (zero between sweeps)

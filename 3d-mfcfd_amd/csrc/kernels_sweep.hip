@@ -132,10 +132,12 @@ constexpr int kSweepWaves = kSweepGroup;
 constexpr int kSweepBlock = 64 * kSweepWaves;
 // the late entries sit on lanes 64 - kMaxLate .. 63, which two row shifts sum
 static_assert(kMaxLate >= 1 && kMaxLate <= 4, "late lanes must fit the last four lanes of a row");
-// doubles per point of pub: a record fills part of one aligned 64-byte (FP64)
-// or 32-byte (mixed) piece of memory
+// record j of pub (T of the kernel) or of dsrc (double)
 template <typename T>
-constexpr long long kPubStride = sizeof(T) == 4 ? 4 : 8;
+__device__ __forceinline__ double* record(double* base, long long j) {
+    static_assert(kRecord<T> % 2 == 0 && 8 % kRecord<T> == 0, "records are polled in aligned 16-byte pieces");
+    return base + kRecord<T> * j;
+}
 // about a second of polling; legitimate waits end within milliseconds
 constexpr int kSpinLimit = 1 << 20;
 // polls by atomic load before the atomic-add fallback
@@ -380,11 +382,11 @@ __device__ __forceinline__ void finish_position(const SweepAsync& a, double* dU,
     // the next position of the chain first
 #pragma unroll
     for (int r = 0; r < NW; ++r) __hip_atomic_store(lds + r, w[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    unsigned long long* pub = reinterpret_cast<unsigned long long*>(a.pub + kPubStride<T> * (long long)i);
+    unsigned long long* pub = reinterpret_cast<unsigned long long*>(record<T>(a.pub, i));
     publish_words<NW>(pub, w);
     if (slot >= 0) {
 #pragma unroll
-        for (int r = 0; r < 5; ++r) store_value(a.dsrc + 5 * (long long)slot + r, res[r]);
+        for (int r = 0; r < 5; ++r) store_value(record<double>(a.dsrc, slot) + r, res[r]);
     }
 #pragma unroll
     for (int r = 0; r < 5; ++r) dU[5 * (long long)i + r] = res[r];
@@ -461,14 +463,13 @@ __global__ void __launch_bounds__(kBlock) k_sweep_snap(DevGeom g, DevState s, co
     }
 }
 
-// pending marks: all of pub, 16 bytes a thread, and every slot of dsrc
+// pending marks: all of pub and every slot of dsrc, 16 bytes a thread
 __global__ void __launch_bounds__(kBlock) k_sweep_mark(SweepAsync a, long long pub_pairs) {
     const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e < pub_pairs) {
         reinterpret_cast<u64x2*>(a.pub)[e] = u64x2{kPending, kPending};
-    } else if (e < pub_pairs + 5LL * a.n_wait_src) {
-        __hip_atomic_store(reinterpret_cast<unsigned long long*>(a.dsrc) + (e - pub_pairs), kPending,
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if (e < pub_pairs + kRecord<double> / 2 * (long long)a.n_wait_src) {
+        reinterpret_cast<u64x2*>(a.dsrc)[e - pub_pairs] = u64x2{kPending, kPending};
     }
 }
 
@@ -526,7 +527,7 @@ __global__ void __launch_bounds__(kSweepBlock, sizeof(T) == 4 ? 4 : 2) k_sweep_a
                 const long long q = (long long)(first >> kTakeShift);
                 double res[5];
                 if (first & kTakeWait) {
-                    wait_state<double>(a.dsrc + 5 * (long long)a.src_slot[q], nullptr, res, a.stalls, a.zero);
+                    wait_state<double>(record<double>(a.dsrc, a.src_slot[q]), nullptr, res, a.stalls, a.zero);
                 } else {
 #pragma unroll
                     for (int r = 0; r < 5; ++r) res[r] = a.dold[5 * q + r];
@@ -575,7 +576,7 @@ __global__ void __launch_bounds__(kSweepBlock, sizeof(T) == 4 ? 4 : 2) k_sweep_a
                     flux_eval<T, true>(dir_family(cls, d), d >> 1, (d & 1) ? -1 : 1, ft, pt, T(fp.pi), Gold);
                     if (SPLIT && late) break;
                     if (packed & kTakeWait) {
-                        wait_state<T>(a.pub + kPubStride<T> * k, nullptr, pt, a.stalls, a.zero);
+                        wait_state<T>(record<T>(a.pub, k), nullptr, pt, a.stalls, a.zero);
                     } else {
 #pragma unroll
                         for (int r = 0; r < 5; ++r) pt[r] = T(a.pold[5 * k + r]);
@@ -596,7 +597,7 @@ __global__ void __launch_bounds__(kSweepBlock, sizeof(T) == 4 ? 4 : 2) k_sweep_a
                 wave_sum5(acc);
                 if (late) {
                     T pt[5], Gnew[5];
-                    wait_state<T>(a.pub + kPubStride<T> * k, from, pt, a.stalls, a.zero);
+                    wait_state<T>(record<T>(a.pub, k), from, pt, a.stalls, a.zero);
                     // on the dependency chain from here to the publication
                     __builtin_amdgcn_s_setprio(3);
                     flux_eval<T, true>(dir_family(cls, d), d >> 1, (d & 1) ? -1 : 1, ft, pt, T(fp.pi), Gnew);
@@ -678,7 +679,8 @@ void launch_one(const DevGeom& g, const DevState& s, const FlowParams& p, const 
     if (n_snap > 0)
         hipLaunchKernelGGL(k_sweep_snap, dim3(grid_for(n_snap, kBlock)), dim3(kBlock), 0, st, g, s,
                            (const double*)dU, a);
-    const long long pairs = kPubStride<T> / 2 * g.n, n_mark = pairs + 5LL * a.n_wait_src;
+    const long long pairs = kRecord<T> / 2 * (long long)g.n;
+    const long long n_mark = pairs + kRecord<double> / 2 * (long long)a.n_wait_src;
     hipLaunchKernelGGL(k_sweep_mark, dim3(grid_for(n_mark, kBlock)), dim3(kBlock), 0, st, a, pairs);
     if (ev) (void)hipEventRecord(ev[0], st);
     if (a.split)

@@ -56,6 +56,12 @@ constexpr int kMaxLate = 4;
 constexpr unsigned kTakeCopy = 7u;
 // positions of a group: one per wave of the sweep kernel's workgroup
 constexpr int kSweepGroup = 8;
+// doubles from one published record of the sweep kernel to the next, five
+// doubles or five floats a record: the kernel polls and publishes it in
+// 16-byte pieces, and counts on each of its 64-bit words coming whole, so every
+// record starts on a 16-byte boundary and stays within one 64-byte line
+template <typename T>
+constexpr int kRecord = sizeof(T) == 4 ? 4 : 8;
 constexpr int kTakeShift = 4;
 
 struct SweepPlanInputs {
