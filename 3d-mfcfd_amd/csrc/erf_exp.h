@@ -420,10 +420,14 @@ __device__ __forceinline__ double scalar(double v) {
 }
 
 // exp(x) by its Taylor series to x^13 on |r| <= ln(2)/2, x = n*ln(2) + r with
-// ln(2) in two parts (n times the first is exact for |n| < 2^11): 0.8 ulp.
-// Results beyond the range of doubles are 0 and infinity; x is not -infinity.
+// ln(2) in two parts (n times the first is exact for |n| < 2^12): 0.8 ulp.
+// Results beyond the range of doubles are 0 and infinity, infinite x included:
+// below -1500, where exp is 0, -1500 takes x's place, since r, and with it the
+// polynomial's sign, would follow x down (a NaN compares false and stays); far
+// above, r and the polynomial grow with x and the result is infinity anyway.
 __device__ __forceinline__ double exp_series(double x) {
-    const double n = __builtin_fmax(__builtin_fmin(__builtin_rint(x * scalar(1.4426950408889634)), 2100.0), -2100.0);
+    x = x < -1500.0 ? -1500.0 : x;
+    const double n = __builtin_fmin(__builtin_rint(x * scalar(1.4426950408889634)), 2100.0);
     double r = fma(n, scalar(-0x1.62e42fefap-1), x);
     r = fma(n, scalar(-0x1.cf79abc9e3b3ap-40), r);
     double a = scalar(1.0 / 6227020800.0);
