@@ -164,8 +164,9 @@ struct mfcfd_ctx {
         DevBuf<int> seq, old_pts, old_src, wait_src;
         DevBuf<long long> take_ptr;
         DevBuf<unsigned> take;
-        DevBuf<unsigned char> late, late_src;
-        DevBuf<int> slots;
+        DevBuf<unsigned char> late;
+        DevBuf<int> slots[2];                // by precision (SweepChains::grouping)
+        DevBuf<unsigned char> late_src[2];
         DevBuf<double> wgt;
         std::vector<int> level_ptr;   // host copy of the level cuts of seq
         int count = 0;
@@ -177,8 +178,8 @@ struct mfcfd_ctx {
             take_ptr.release();
             take.release();
             late.release();
-            late_src.release();
-            slots.release();
+            for (auto& b : slots) b.release();
+            for (auto& b : late_src) b.release();
             wgt.release();
             level_ptr.clear();
             count = 0;
@@ -215,7 +216,7 @@ struct mfcfd_ctx {
     hipGraphExec_t graph_exec = nullptr;
     bool graph_stale = true;
     int sweep_grid = 0, sweep_grid_mixed = 0;
-    int sweep_chain[2] = {1, 1};   // longest chain of the sweep groups, by precision
+    SweepChains sweep_chains;
     // bookkeeping of fpi_solver.f90:38-43
     double res_old = 0.0, res_new = 0.0, residue = 0.0, max_res = 0.0, sum_res_sqr = 0.0;
     int max_res_point = 0, last_t = 0;
@@ -432,9 +433,10 @@ SweepAsync sweep_args(mfcfd_ctx* c, mfcfd_ctx::DevSweepDir& d) {
     a.take_ptr = d.take_ptr.p;
     a.take = d.take.p;
     a.late = d.late.p;
-    a.slots = d.slots.p;
-    a.late_src = d.late_src.p;
-    a.groups = (int)(d.slots.n / kSweepGroup);
+    const int by = c->sweep_chains.grouping(c->fp.mixed);
+    a.slots = by >= 0 ? d.slots[by].p : nullptr;
+    a.late_src = by >= 0 ? d.late_src[by].p : nullptr;
+    a.groups = (d.count + kSweepGroup - 1) / kSweepGroup;
     a.wgt = d.wgt.p;
     a.old_pts = d.old_pts.p;
     a.n_old = (int)d.old_pts.n;
@@ -450,7 +452,7 @@ SweepAsync sweep_args(mfcfd_ctx* c, mfcfd_ctx::DevSweepDir& d) {
     a.ctr = c->sweep_ctr.p;
     a.stalls = &c->rec.p->stalls;
     a.zero = 0;
-    a.split = c->sweep_chain[c->fp.mixed] > 1;
+    a.split = by >= 0;
     return a;
 }
 
@@ -501,22 +503,6 @@ int do_sweeps(mfcfd_ctx* c) {
     return launch_error("implicit sweeps");
 }
 
-// Longest chain of positions a sweep workgroup hands from wave to wave, from
-// the waves resident on the chip and the plan's mean positions per dependency
-// level.  A chain shortens the path through the levels, and holds all eight
-// waves of its workgroup until its last position is done: with many levels in
-// flight that costs nothing, with few it keeps ready positions waiting.  Sweep
-// kernel times, in ms, with chains of 1 (late entries not set apart), 2 and 8:
-//   1M FP64, 13.6 levels in flight    11.4   9.7   9.2
-//   3M FP64, 6.8                      20.5  18.0  18.9
-//   8M FP64, 4.1                      33.8  35.4  41.5
-//   3M mixed, 13.6                    17.5  13.4  12.9
-//   8M mixed, 8.2                     26.8  22.5  23.5
-int chain_for(int resident_waves, double per_level) {
-    const double levels = resident_waves / std::max(per_level, 1.0);
-    return levels >= 12.0 ? kSweepGroup : levels >= 6.0 ? 2 : 1;
-}
-
 // Builds the LU-SGS plan of the given implicit form (SweepPlan) from the
 // host copies kept at bind, uploads it and computes every entry's weight.
 // Synchronous; never called while a graph is being captured.
@@ -561,11 +547,22 @@ int build_plan(mfcfd_ctx* c, int form) {
                              kSweepGroup * sweep_async_grid(n, c->params.power == 0.0, true)};
     const double per_level = 2.0 * (double)plan.fwd.seq.size() /
                              std::max<double>(1.0, (double)(plan.fwd.level_ptr.size() + plan.bwd.level_ptr.size()) - 2.0);
-    for (int m = 0; m < 2; ++m) c->sweep_chain[m] = chain_for(resident[m], per_level);
-    const int chain = c->sweep_chain[c->fp.mixed];
-    std::future<void> f = std::async([&] { group_positions(plan.fwd, n, chain); });
-    group_positions(plan.bwd, n, chain);
-    f.get();
+    // the groups of both precisions now, side by side: a precision set later
+    // must not have to build any (mfcfd_run_noalloc, graph capture)
+    for (int m = 0; m < 2; ++m) c->sweep_chains.chain[m] = chain_for(resident[m], per_level);
+    std::vector<int> slots[2][2];   // [direction][precision]
+    std::vector<unsigned char> late_src[2][2];
+    {
+        std::vector<std::future<void>> work;
+        for (int dir = 0; dir < 2; ++dir)
+            for (int m = 0; m < 2; ++m)
+                if (c->sweep_chains.grouping(m) == m)
+                    work.push_back(std::async([&, dir, m] {
+                        group_positions(dir == 0 ? plan.fwd : plan.bwd, n, c->sweep_chains.chain[m], slots[dir][m],
+                                        late_src[dir][m]);
+                    }));
+        for (auto& w : work) w.get();
+    }
     hipStream_t st = c->stream;
     c->sw_fwd.release();
     c->sw_bwd.release();
@@ -585,10 +582,11 @@ int build_plan(mfcfd_ctx* c, int form) {
         const unsigned char none_c = 0;
         if ((r = upload(d.late, pd.late.empty() ? &none_c : pd.late.data(), std::max<size_t>(pd.late.size(), 1), st)))
             return r;
-        if ((r = upload(d.late_src, pd.late_src.empty() ? &none_c : pd.late_src.data(),
-                        std::max<size_t>(pd.late_src.size(), 1), st)))
-            return r;
-        if ((r = upload(d.slots, pd.slots.data(), pd.slots.size(), st))) return r;
+        const int dir = &pd == &plan.fwd ? 0 : 1;
+        for (int m = 0; m < 2; ++m) {
+            if ((r = upload(d.slots[m], slots[dir][m].data(), slots[dir][m].size(), st))) return r;
+            if ((r = upload(d.late_src[m], late_src[dir][m].data(), late_src[dir][m].size(), st))) return r;
+        }
         if (d.wgt.alloc(std::max<size_t>(pd.take.size(), 1)) != hipSuccess)
             return fail(MFCFD_ENOMEM, "sweep weights (%zu entries)", pd.take.size());
         if ((r = upload(d.old_pts, pd.old_pts.data(), pd.old_pts.size(), st))) return r;
@@ -625,7 +623,7 @@ int build_plan(mfcfd_ctx* c, int form) {
     launch_sweep_weights(c->geom(), sweep_args(c, c->sw_bwd), c->fp.power, st);
     if ((rc = launch_error("sweep weights"))) return rc;
     HIP_TRY(hipStreamSynchronize(st));   // the host plan ends here
-    const int groups = (int)(std::max(plan.fwd.slots.size(), plan.bwd.slots.size()) / kSweepGroup);
+    const int groups = (std::max(c->sw_fwd.count, c->sw_bwd.count) + kSweepGroup - 1) / kSweepGroup;
     c->sweep_grid = sweep_async_grid(groups, c->params.power == 0.0, false);
     c->sweep_grid_mixed = sweep_async_grid(groups, c->params.power == 0.0, true);
     c->plan_form = form;

@@ -61,10 +61,10 @@ struct SweepAsync {
     const unsigned* take;       // k << 4 | wait << 3 | direction (7: supersonic copy) of every taken entry
     const unsigned char* late;  // [count]: position t's last late[t] entries read the wait dependency
                                 // that executes last (at most 4; 0: none set apart)
-    const int* slots;           // [kSweepGroup*groups] position of each wave of a group (-1: none); not
-                                // read when split is 0
+    const int* slots;           // [kSweepGroup*groups] position of each wave of a group (-1: none); null
+                                // when split is 0
     const unsigned char* late_src;  // [count]: 1 + the wave of the same group that executes the point of
-                                // position t's late entries, 0: another group's
+                                // position t's late entries, 0: another group's; null when split is 0
     int groups;
     int split;                  // 1: groups of chains, late entries summed after the others; 0: groups of
                                 // consecutive positions, every entry waited for together (same sums)

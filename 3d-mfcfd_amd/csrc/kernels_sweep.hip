@@ -549,7 +549,7 @@ __global__ void __launch_bounds__(kSweepBlock, sizeof(T) == 4 ? 4 : 2) k_sweep_a
             // end of the list, at most kMaxLate of them, on the wave's last
             // lanes; the others share the lanes below.
             const int n_late = __builtin_amdgcn_readfirstlane((int)a.late[t]);
-            const int src = __builtin_amdgcn_readfirstlane((int)a.late_src[t]);
+            const int src = SPLIT ? __builtin_amdgcn_readfirstlane((int)a.late_src[t]) : 0;
             const unsigned long long* from = src ? sh_pub[round & 1][src - 1] : nullptr;
             const int stride = 64 - n_late;
             const bool late = lane >= stride;

@@ -248,10 +248,11 @@ int build_dir(const SweepPlanInputs& in, bool forward, SweepDirPlan& out) {
 
 }  // namespace
 
-void group_positions(SweepDirPlan& plan, int n, int max_chain) {
+void group_positions(const SweepDirPlan& plan, int n, int max_chain, std::vector<int>& slots,
+                     std::vector<unsigned char>& late_src) {
     const int m = (int)plan.seq.size();
-    plan.slots.clear();
-    plan.late_src.assign(m, 0);
+    slots.clear();
+    late_src.assign(m, 0);
     std::vector<int> at(n, -1);
     for (int u = 0; u < m; ++u) at[plan.seq[u]] = u;
     // height: the longest chain of dependents below a position; joins: the
@@ -269,12 +270,12 @@ void group_positions(SweepDirPlan& plan, int n, int max_chain) {
         if (j < 0 || height[u] > height[j]) j = u;
     }
     std::vector<char> placed(m, 0);
-    plan.slots.reserve((size_t)m + kSweepGroup);
+    slots.reserve((size_t)m + kSweepGroup);
     for (int u = 0; u < m; ++u) {
         if (placed[u]) continue;
         placed[u] = 1;
-        plan.slots.push_back(u);
-        for (int tail = u, len = 1; len < max_chain && plan.slots.size() % kSweepGroup != 0; ++len) {
+        slots.push_back(u);
+        for (int tail = u, len = 1; len < max_chain && slots.size() % kSweepGroup != 0; ++len) {
             const int v = joins[tail];
             if (v < 0) break;
             bool ready = true;
@@ -282,12 +283,17 @@ void group_positions(SweepDirPlan& plan, int n, int max_chain) {
                 if (plan.take[e] & kTakeWait) ready = placed[at[plan.take[e] >> kTakeShift]];
             if (!ready) break;
             placed[v] = 1;
-            plan.late_src[v] = (unsigned char)(1 + (plan.slots.size() - 1) % kSweepGroup);
-            plan.slots.push_back(v);
+            late_src[v] = (unsigned char)(1 + (slots.size() - 1) % kSweepGroup);
+            slots.push_back(v);
             tail = v;
         }
     }
-    while (plan.slots.size() % kSweepGroup != 0) plan.slots.push_back(-1);
+    while (slots.size() % kSweepGroup != 0) slots.push_back(-1);
+}
+
+int chain_for(int resident_waves, double per_level) {
+    const double levels = resident_waves / std::max(per_level, 1.0);
+    return levels >= 12.0 ? kSweepGroup : levels >= 6.0 ? 2 : 1;
 }
 
 int SweepPlan::build(const SweepPlanInputs& in) {

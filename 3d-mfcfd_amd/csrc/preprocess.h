@@ -104,7 +104,33 @@ struct SweepPlan {
 // group therefore never waits for a later one, and inside it positions wait
 // only for earlier positions, so groups taken in order always finish,
 // however few of them run at a time.
-void group_positions(SweepDirPlan& plan, int n, int max_chain);
+void group_positions(const SweepDirPlan& plan, int n, int max_chain, std::vector<int>& slots,
+                     std::vector<unsigned char>& late_src);
+inline void group_positions(SweepDirPlan& plan, int n, int max_chain) {
+    group_positions(plan, n, max_chain, plan.slots, plan.late_src);
+}
+
+// Longest chain of positions a sweep workgroup hands from wave to wave, from
+// the waves resident on the chip and the plan's mean positions per dependency
+// level.  A chain shortens the path through the levels, and holds all eight
+// waves of its workgroup until its last position is done: with many levels in
+// flight that costs nothing, with few it keeps ready positions waiting.  Sweep
+// kernel times, in ms, with chains of 1 (late entries not set apart), 2 and 8:
+//   1M FP64, 13.6 levels in flight    11.4   9.7   9.2
+//   3M FP64, 6.8                      20.5  18.0  18.9
+//   8M FP64, 4.1                      33.8  35.4  41.5
+//   3M mixed, 13.6                    17.5  13.4  12.9
+//   8M mixed, 8.2                     26.8  22.5  23.5
+int chain_for(int resident_waves, double per_level);
+
+// Chains of the two precisions (0: FP64, 1: mixed) of one bound context, which
+// may change its precision at any time: each has its groups.
+struct SweepChains {
+    int chain[2] = {1, 1};
+    // the precision whose groups precision m runs (its own, or the other's
+    // when the chains are alike); -1: consecutive positions, no groups
+    int grouping(int m) const { return chain[m] == 1 ? -1 : m == 1 && chain[0] == chain[1] ? 0 : m; }
+};
 
 // the list a sweep walks for point i and direction d (device numbers):
 // the flux stencil's list, except that a wall point takes no ZPOS term and
