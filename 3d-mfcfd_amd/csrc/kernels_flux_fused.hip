@@ -26,6 +26,8 @@
 // point's q, qm and dq were fetched from HBM about 19 times per launch.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device_common.h"
 #include "device_state.h"
 #include "erf_exp.h"
@@ -410,24 +412,26 @@ void launch_class(const DevGeom& g, const DevState& s, const FlowParams& p, cons
         hipLaunchKernelGGL((k_flux_fused<CLASS, false, T, 2>), grid, blk, lds, st, g, s, p, idx, count);
         return;
     }
-    switch (ks.waves) {
-        case 1: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 1>), grid, blk, lds, st, g, s, p, idx, count); break;
-        case 3: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 3>), grid, blk, lds, st, g, s, p, idx, count); break;
-        case 4: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 4>), grid, blk, lds, st, g, s, p, idx, count); break;
-        case 5:
-            if constexpr (sizeof(T) == 4) {
-                hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 5>), grid, blk, lds, st, g, s, p, idx, count);
-                break;
-            }
-            [[fallthrough]];
-        case 6:
-            if constexpr (sizeof(T) == 4) {
-                hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 6>), grid, blk, lds, st, g, s, p, idx, count);
-                break;
-            }
-            [[fallthrough]];
-        default: hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 2>), grid, blk, lds, st, g, s, p, idx, count); break;
+    // caps of three waves and more are the FP32 variants'; the FP64 kernels spill
+    // under them (2M points, interior class: 2.88 ms with three and 5.09 with four
+    // against 1.95 with two) and run with two instead
+    if constexpr (sizeof(T) == 4) {
+        const auto launch = [&](auto waves) {
+            hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, decltype(waves)::value>), grid, blk, lds, st, g, s, p, idx,
+                               count);
+        };
+        switch (ks.waves) {
+            case 3: return launch(std::integral_constant<int, 3>{});
+            case 4: return launch(std::integral_constant<int, 4>{});
+            case 5: return launch(std::integral_constant<int, 5>{});
+            case 6: return launch(std::integral_constant<int, 6>{});
+            default: break;
+        }
     }
+    if (ks.waves == 1)
+        hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 1>), grid, blk, lds, st, g, s, p, idx, count);
+    else
+        hipLaunchKernelGGL((k_flux_fused<CLASS, true, T, 2>), grid, blk, lds, st, g, s, p, idx, count);
 }
 
 }  // namespace

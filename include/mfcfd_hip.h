@@ -227,12 +227,12 @@ int mfcfd_run_graph(mfcfd_ctx *ctx, int t0, int n_iters, double *res_new_hist, d
  * bound cloud(s) and the current state, every compiled variant of the
  * gather kernels -- block size 64/128/256 x minimum waves per SIMD (the
  * register cap: 2/4/6 for the mixed q-derivative kernel, whose FP64 form has one
- * variant, 1..4 for the fused flux
- * kernels, 1..6 for their mixed-precision FP32 variants), then for the chosen shape an LDS reservation that caps the
- * resident waves per CU (fewer points in flight per XCD keep their
- * neighbours in that XCD's L2) -- and, in implicit mode, the sync-free
- * sweeps on 1, 1/2 or 1/4 of the resident grid; keeps the fastest.  Results do not depend on the
- * shapes.  It recomputes U, q, qm, dq, delt, flux_res and (implicit)
+ * variant; 1..6 for the mixed-precision fused flux kernels, 1 and 2 for the FP64
+ * ones, where higher caps are accepted and mean 2), then for the chosen shape an
+ * LDS reservation that caps the resident waves per CU (fewer points in flight
+ * per XCD keep their neighbours in that XCD's L2) -- and, in implicit mode, the
+ * sync-free sweeps on 1, 1/2, 1/4 or 1/8 of the resident grid; keeps the
+ * fastest.  Results do not depend on the shapes.  It recomputes U, q, qm, dq, delt, flux_res and (implicit)
  * delUp/delUn from prim as one iteration's first steps would; prim is not
  * touched. */
 typedef struct mfcfd_tuning {
