@@ -1742,42 +1742,45 @@ int mfcfd_autotune(mfcfd_ctx* c, int repeats, mfcfd_tuning* out) {
         launch_timestep(g, s, c->fp, c->stream);
     }
     if (c->params.flux_order == MFCFD_FLUX_FUSED) {
+        // The joint launch has one shape, whatever is asked for: its time is
+        // reported, and shape 256 with waves 0 (the default).  Class launches:
         // FP32 variants come capped at up to 6 waves per SIMD (a few spilled
-        // registers for more resident waves), FP64 ones at 1 and 2
-        const std::vector<int> waves = c->fp.mixed ? std::vector<int>{1, 2, 3, 4, 5, 6} : std::vector<int>{1, 2};
+        // registers for more resident waves), FP64 ones at 1 and 2, weighted
+        // ones (power != 0) at 2.
+        const bool joint = flux_joint(c->tl, c->fp.power);
+        const std::vector<int> waves = joint                 ? std::vector<int>{}
+                                       : c->fp.power != 0.0 ? std::vector<int>{2}
+                                       : c->fp.mixed        ? std::vector<int>{1, 2, 3, 4, 5, 6}
+                                                            : std::vector<int>{1, 2};
         for (int part = 1; part <= 2; ++part) {
             const int count = part == 1 ? c->tl.n_fused_interior : c->tl.n_fused_wall;
             if (count == 0) continue;
-            double best_ms = 1e30;
-            KernelShape pick;
-            for (int bl : blocks)
-                for (int w : waves) {
-                    LaunchShapes ls = best;
-                    (part == 1 ? ls.flux_interior : ls.flux_wall) = KernelShape{bl, w};
-                    double ms = 0.0;
-                    if ((rc = time_launches(c, repeats, pre_f,
-                                            [&] { launch_flux_residual(g, s, c->fp, c->tl, c->stream, part, ls); },
-                                            &ms)))
-                        return rc;
-                    if (bl == 256 && w == 2) (part == 1 ? t.flux_interior_default_ms : t.flux_wall_default_ms) = ms;
-                    if (ms < best_ms) {
-                        best_ms = ms;
-                        pick = KernelShape{bl, w};
-                    }
-                }
-            for (int lds : caps(pick.block, {4, 6, 8, 12})) {
+            auto time_shape = [&](const KernelShape& ks, double* ms) {
                 LaunchShapes ls = best;
-                KernelShape ks = pick;
-                ks.lds = lds;
                 (part == 1 ? ls.flux_interior : ls.flux_wall) = ks;
+                return time_launches(c, repeats, pre_f,
+                                     [&] { launch_flux_residual(g, s, c->fp, c->tl, c->stream, part, ls); }, ms);
+            };
+            KernelShape pick{256, joint ? 0 : 2};
+            double best_ms = 0.0;
+            if ((rc = time_shape(pick, &best_ms))) return rc;
+            (part == 1 ? t.flux_interior_default_ms : t.flux_wall_default_ms) = best_ms;
+            auto attempt = [&](const KernelShape& ks) {
                 double ms = 0.0;
-                if ((rc = time_launches(c, repeats, pre_f,
-                                        [&] { launch_flux_residual(g, s, c->fp, c->tl, c->stream, part, ls); }, &ms)))
-                    return rc;
-                if (ms < best_ms) {
+                const int r = time_shape(ks, &ms);
+                if (!r && ms < best_ms) {
                     best_ms = ms;
                     pick = ks;
                 }
+                return r;
+            };
+            for (int bl : blocks)
+                for (int w : waves)
+                    if (!(bl == 256 && w == 2) && (rc = attempt(KernelShape{bl, w}))) return rc;
+            if (!joint) {
+                const KernelShape bare = pick;
+                for (int lds : caps(bare.block, {4, 6, 8, 12}))
+                    if ((rc = attempt(KernelShape{bare.block, bare.waves, lds}))) return rc;
             }
             (part == 1 ? best.flux_interior : best.flux_wall) = pick;
             (part == 1 ? t.flux_interior_ms : t.flux_wall_ms) = best_ms;

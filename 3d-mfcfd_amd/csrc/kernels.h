@@ -31,7 +31,7 @@ struct KernelShape {
     int lds = 0;   // dynamic LDS bytes reserved per block: caps the blocks resident per CU
 };
 // shapes the autotuner chooses (defaults until it runs); the flux shapes are
-// those of a launch per class (flux_small in kernels_flux_fused.hip)
+// those of a launch per class, without effect where flux_joint
 struct LaunchShapes {
     KernelShape flux_interior, flux_wall, qderiv;
     int sweep_div = 1;   // sync-free sweeps use the resident grid / sweep_div
@@ -115,6 +115,9 @@ constexpr int kFluxAll = 7;
 void launch_flux_residual(const DevGeom& g, const DevState& s, const FlowParams& p,
                           const TypeLists& tl, hipStream_t st, int parts = kFluxAll,
                           const LaunchShapes& ls = LaunchShapes());
+// one launch takes both classes of the fused flux (a cloud that does not fill
+// the chip) rather than one each
+bool flux_joint(const TypeLists& tl, double power);
 // reference-order flux residual of every point of a class (parity path)
 void launch_flux_residual_reference(const DevGeom& g, const DevState& s, const FlowParams& p,
                                     const TypeLists& tl, hipStream_t st);

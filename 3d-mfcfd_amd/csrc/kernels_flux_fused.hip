@@ -454,14 +454,17 @@ void launch_class(const DevGeom& g, const DevState& s, const FlowParams& p, cons
 //   150,000                384 -> 336            229 -> 205   (4 + 4)
 //   500,000               1120 -> 1057           635 -> 625   (4 + 4)
 //   1,000,000 together    2197 -> 2132          1262 -> 1289: a launch each
+bool flux_joint(const TypeLists& tl, double power) {
+    const int ng = tl.n_fused_wall, ni = tl.n_fused_interior;
+    return ng <= (power != 0.0 ? 20000 : 100000) && ni <= 450000;
+}
 template <typename T>
 static bool flux_small(const DevGeom& g, const DevState& s, const FlowParams& p, const TypeLists& tl,
                        hipStream_t st, int parts) {
+    if (!flux_joint(tl, p.power)) return false;
     const int ng = tl.n_fused_wall, ni = tl.n_fused_interior;
-    if (ng > 100000 || ni > 450000) return false;
     if (p.power != 0.0) {
         // weighted least squares: the two that cover most sizes
-        if (ng > 20000) return false;
         if (ni > 24000) launch_small<false, T, 16, 4>(g, s, p, tl, parts, st);
         else launch_small<false, T, 16, 16>(g, s, p, tl, parts, st);
     } else if (ng > 20000) {

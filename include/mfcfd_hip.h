@@ -232,9 +232,14 @@ int mfcfd_run_graph(mfcfd_ctx *ctx, int t0, int n_iters, double *res_new_hist, d
  * LDS reservation that caps the resident waves per CU (fewer points in flight
  * per XCD keep their neighbours in that XCD's L2) -- and, in implicit mode, the
  * sync-free sweeps on 1, 1/2, 1/4 or 1/8 of the resident grid; keeps the
- * fastest.  Results do not depend on the shapes.  It recomputes U, q, qm, dq, delt, flux_res and (implicit)
- * delUp/delUn from prim as one iteration's first steps would; prim is not
- * touched. */
+ * fastest.  Results do not depend on the shapes.
+ * Up to 450,000 points of the fused interior class and 100,000 of the general
+ * class (mfcfd_point_classes; 20,000 with power != 0) one launch takes both and
+ * has one shape: flux shapes are accepted and without effect there, and the
+ * autotuner reports block 256, waves 0 (the default) and no LDS for them, with
+ * that launch's times as both the chosen and the default shape's.
+ * It recomputes U, q, qm, dq, delt, flux_res and (implicit) delUp/delUn from prim
+ * as one iteration's first steps would; prim is not touched. */
 typedef struct mfcfd_tuning {
     int flux_interior_block, flux_interior_waves;
     int flux_wall_block, flux_wall_waves;
@@ -245,7 +250,7 @@ typedef struct mfcfd_tuning {
     double flux_interior_default_ms, flux_wall_default_ms, qderiv_default_ms, sweeps_default_ms;
 } mfcfd_tuning;
 int mfcfd_autotune(mfcfd_ctx *ctx, int repeats, mfcfd_tuning *out);
-/* apply shapes chosen earlier (times ignored) */
+/* apply shapes chosen earlier (times ignored; 0: the default) */
 int mfcfd_set_tuning(mfcfd_ctx *ctx, const mfcfd_tuning *in);
 
 int mfcfd_get_residual(mfcfd_ctx *ctx, mfcfd_residual *out);

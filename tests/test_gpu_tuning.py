@@ -45,3 +45,31 @@ def test_every_class_launch_variant_agrees(large, precision, shapes):
             want = got
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     s.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_autotuner_reports_the_joint_launch_as_the_default(precision):
+    """One launch takes both classes of a small cloud, whatever the shapes:
+    there is nothing to choose, and no time of a shape that never ran."""
+    cl = shells(30000)
+    print(f"[gpu] autotune {precision}, {cl.n} points", flush=True)
+    s = solver.Solver(cl, 0.6, 2.0, 0.2, precision=precision)
+    s.upload("prim", np.tile(pc.freestream_prim(0.6, 2.0), (cl.n, 1)))
+    t = s.autotune(2)
+    s.close()
+    for part in ("flux_interior", "flux_wall"):
+        assert (t[f"{part}_block"], t[f"{part}_waves"], t[f"{part}_lds"]) == (256, 0, 0)
+        assert 0.0 < t[f"{part}_ms"] == t[f"{part}_default_ms"]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_autotuner_chooses_among_the_class_launches(large, precision):
+    print(f"[gpu] autotune {precision}, {large.n} points", flush=True)
+    s = solver.Solver(large, 0.6, 2.0, 0.2, precision=precision)
+    s.upload("prim", np.tile(pc.freestream_prim(0.6, 2.0), (large.n, 1)))
+    t = s.autotune(1)
+    s.close()
+    for part in ("flux_interior", "flux_wall"):
+        assert t[f"{part}_block"] in (64, 128, 256)
+        assert 1 <= t[f"{part}_waves"] <= (2 if precision == "fp64" else 6)
+        assert 0.0 < t[f"{part}_ms"] <= t[f"{part}_default_ms"]
