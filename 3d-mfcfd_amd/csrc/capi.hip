@@ -1707,33 +1707,33 @@ int mfcfd_autotune(mfcfd_ctx* c, int repeats, mfcfd_tuning* out) {
     };
     LaunchShapes best = c->shapes;
     if (c->fp.inner_iterations == 0) {
-        const int waves[3] = {2, 4, 6};
-        double best_ms = 1e30;
-        for (int bl : blocks)
-            for (int w : waves) {
-                KernelShape ks;
-                ks.block = bl;
-                ks.waves = w;
-                double ms = 0.0;
-                if ((rc = time_launches(c, repeats, pre_q, [&] { launch_qderiv_timestep(g, s, c->fp, c->stream, ks); }, &ms)))
-                    return rc;
-                if (bl == 256 && w == 4) t.qderiv_default_ms = ms;
-                if (ms < best_ms) {
-                    best_ms = ms;
-                    best.qderiv = ks;
-                }
-            }
-        for (int lds : caps(best.qderiv.block, {8, 12, 16})) {
-            KernelShape ks = best.qderiv;
-            ks.lds = lds;
+        // the FP64 form and the weighted one (power != 0) have one register cap
+        const KernelShape def = qderiv_default(c->fp.mixed != 0);
+        const std::vector<int> waves = c->fp.mixed && c->fp.power == 0.0 ? std::vector<int>{2, 4, 6}
+                                                                         : std::vector<int>{def.waves};
+        double best_ms = 0.0;
+        auto time_shape = [&](const KernelShape& ks, double* ms) {
+            return time_launches(c, repeats, pre_q, [&] { launch_qderiv_timestep(g, s, c->fp, c->stream, ks); }, ms);
+        };
+        best.qderiv = def;
+        if ((rc = time_shape(def, &best_ms))) return rc;
+        t.qderiv_default_ms = best_ms;
+        auto attempt = [&](const KernelShape& ks) {
+            if (ks.block == def.block && ks.waves == def.waves && ks.lds == def.lds) return 0;
             double ms = 0.0;
-            if ((rc = time_launches(c, repeats, pre_q, [&] { launch_qderiv_timestep(g, s, c->fp, c->stream, ks); }, &ms)))
-                return rc;
-            if (ms < best_ms) {
+            const int r = time_shape(ks, &ms);
+            if (!r && ms < best_ms) {
                 best_ms = ms;
                 best.qderiv = ks;
             }
-        }
+            return r;
+        };
+        for (int bl : blocks)
+            for (int w : waves)
+                if ((rc = attempt(KernelShape{bl, w}))) return rc;
+        const KernelShape bare = best.qderiv;
+        for (int lds : caps(bare.block, {8, 12, 16}))
+            if ((rc = attempt(KernelShape{bare.block, bare.waves, lds}))) return rc;
         t.qderiv_ms = best_ms;
         best_for_pre = best;
         launch_qderiv_timestep(g, s, c->fp, c->stream, best.qderiv);

@@ -110,6 +110,8 @@ void launch_q_derivatives(const DevGeom& g, const DevState& s, const FlowParams&
 void launch_timestep(const DevGeom& g, const DevState& s, const FlowParams& p, hipStream_t st);
 void launch_qderiv_timestep(const DevGeom& g, const DevState& s, const FlowParams& p, hipStream_t st,
                             const KernelShape& ks = KernelShape());
+// the shape a default-constructed KernelShape stands for there
+KernelShape qderiv_default(bool mixed);
 // flux_residual.f90; part bit 0: fused interior, bit 1: fused wall, bit 2: list-by-list
 constexpr int kFluxAll = 7;
 void launch_flux_residual(const DevGeom& g, const DevState& s, const FlowParams& p,

@@ -1182,21 +1182,24 @@ void launch_timestep(const DevGeom& g, const DevState& s, const FlowParams& p, h
     hipLaunchKernelGGL((k_qderiv_timestep<false, true, true, double>), dim3(grid_for((long long)g.n * kQdGroup, kBlock)),
                        dim3(kBlock), 0, st, g, s, p);
 }
+// The mixed form's 81 registers would let six waves share a SIMD; the points
+// they hold overflow their XCD's L2.  Unless a shape was chosen, 40 KB of LDS per
+// workgroup keep it to four (2M cloud 474 -> 442 us, 600,000 points 136 -> 128; the
+// FP64 form's three waves: no difference).
+KernelShape qderiv_default(bool mixed) { return mixed ? KernelShape{kBlock, 4, 40 * 1024} : KernelShape{kBlock, 2, 0}; }
+
 template <typename QT>
 void launch_qdt(const DevGeom& g, const DevState& s, const FlowParams& p, hipStream_t st, const KernelShape& ks) {
-    int block = ks.block > 0 && ks.block <= kBlock ? ks.block : kBlock;
+    const KernelShape def = qderiv_default(sizeof(QT) == 4);
+    int block = ks.block > 0 && ks.block <= kBlock ? ks.block : def.block;
     block -= block % kQdGroup;
     const dim3 grid(grid_for((long long)g.n * kQdGroup, block)), blk(block);
-    // The mixed form's 81 registers would let six waves share a SIMD; the points
-    // they hold overflow their XCD's L2.  Unless a shape was chosen, 40 KB of
-    // LDS per workgroup keep it to four (2M cloud 474 -> 442 us, 600,000 points
-    // 136 -> 128; the FP64 form's three waves: no difference).
-    const int lds = ks.block > 0 ? ks.lds : sizeof(QT) == 4 ? 40 * 1024 : 0;
+    const int lds = ks.block > 0 || ks.lds > 0 ? ks.lds : def.lds;
     if (p.power != 0.0) {
         hipLaunchKernelGGL((k_qderiv_timestep<true, true, false, QT>), grid, blk, lds, st, g, s, p);
         return;
     }
-    // the FP64 form has one variant: caps at four and six waves spill
+    // the FP64 form has one variant, for two waves: caps at four and six spill
     if constexpr (sizeof(QT) == 4) {
         if (ks.waves == 2 || ks.waves == 6) {
             if (ks.waves == 2)

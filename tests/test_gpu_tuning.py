@@ -73,3 +73,28 @@ def test_autotuner_chooses_among_the_class_launches(large, precision):
         assert t[f"{part}_block"] in (64, 128, 256)
         assert 1 <= t[f"{part}_waves"] <= (2 if precision == "fp64" else 6)
         assert 0.0 < t[f"{part}_ms"] <= t[f"{part}_default_ms"]
+
+
+@pytest.mark.parametrize("precision,power,waves", [("fp64", 0.0, {2}), ("fp64", 2.0, {2}), ("mixed", 0.0, {2, 4, 6}),
+                                                   ("mixed", 2.0, {4})])
+def test_autotuner_starts_from_the_default_q_derivatives(precision, power, waves):
+    """The forms with one register cap report that one, and the default's time
+    is that of the shape that runs by default: the tuned and the default shape
+    agree in every result, and the choice is not slower than the default."""
+    cl = pc.fixture_cloud(3000, seed=6, order="morton", k=25 if power == 0.0 else 22)
+    print(f"[gpu] autotune {precision}, power {power}, {cl.n} points", flush=True)
+    prim = np.tile(pc.freestream_prim(0.6, 2.0), (cl.n, 1))
+    s = solver.Solver(cl, 0.6, 2.0, 0.2, precision=precision, power=power)
+    s.upload("prim", prim)
+    s.run(1, 2)
+    want = s.download("dq")
+    t = s.autotune(2)
+    assert t["qderiv_block"] in (64, 128, 256) and t["qderiv_waves"] in waves
+    assert 0.0 < t["qderiv_ms"] <= t["qderiv_default_ms"]
+    for lds in (t["qderiv_lds"], 0, 65536):
+        for block in (0, t["qderiv_block"]):
+            s.set_tuning({**t, "qderiv_block": block, "qderiv_lds": lds})
+            s.upload("prim", prim)
+            s.run(1, 2)
+            assert np.array_equal(s.download("dq"), want)
+    s.close()
