@@ -596,6 +596,8 @@ int build_plan(mfcfd_ctx* c, int form) {
     };
     if ((rc = put(c->sw_fwd, plan.fwd))) return rc;
     if ((rc = put(c->sw_bwd, plan.bwd))) return rc;
+    // FP64's records whichever precision is set, twice the mixed form's: a
+    // precision set later finds them (mfcfd_run_noalloc)
     if (c->pub.n == 0 && c->pub.alloc_fine((size_t)kRecord<double> * n) != hipSuccess)
         return fail(MFCFD_ENOMEM, "sweep values (fine-grained)");
     // copy sources read as this sweep's delU: a slot each in dsrc
@@ -1716,7 +1718,8 @@ int mfcfd_autotune(mfcfd_ctx* c, int repeats, mfcfd_tuning* out) {
             return time_launches(c, repeats, pre_q, [&] { launch_qderiv_timestep(g, s, c->fp, c->stream, ks); }, ms);
         };
         best.qderiv = def;
-        if ((rc = time_shape(def, &best_ms))) return rc;
+        // twice: the first kernel timed here meets a chip that may have been idle
+        if ((rc = time_shape(def, &best_ms)) || (rc = time_shape(def, &best_ms))) return rc;
         t.qderiv_default_ms = best_ms;
         auto attempt = [&](const KernelShape& ks) {
             if (ks.block == def.block && ks.waves == def.waves && ks.lds == def.lds) return 0;
