@@ -1,9 +1,10 @@
 """Build libmfcfd_hip.so (gfx950) in-tree with hipcc.
 
 Every HIP translation unit is compiled for gfx950 only, with packed FP32
-instructions disabled; the FP64 parity kernels additionally use
--ffp-contract=off so no multiply-add is fused that the reference does not
-fuse.  The sync-free sweeps and the fused flux kernel are the exceptions:
+instructions disabled, and with -ffp-contract=off, so that no multiply-add is
+fused unless the source says so (the q-derivatives and the time step do; the
+rest of the parity kernels keeps the reference's rounding).  The sync-free
+sweeps and the fused flux kernel are the exceptions:
 their own forms of the split fluxes already round differently from the
 reference, so they fuse the multiply-adds within an expression
 (-ffp-contract=on), the same way at every call site.  Objects go to

@@ -9,21 +9,24 @@
 // with a membership bit per direction list, then the list entries that are
 // not an in-order subsequence of conn), reconstructs each end
 // once, evaluates the exponentials and error functions of each axis once
-// per end, and forms the directional fluxes of that edge from them.  Every
-// flux value is computed with the reference's own expressions, so it is
-// bit-identical to the list-by-list kernel; only the least-squares solve is
-// applied edge by edge, through the Cramer weights of each list
-// (sum_j (G_k - G_i)*(c . (dels, delt, deln)) instead of the 3x3 solve of the
-// accumulated sums), which changes the rounding, not the mathematics.
+// per end, and forms the directional fluxes of that edge from them.  The
+// mathematics is the reference's, the rounding is not that of the list-by-list
+// kernel, which keeps the reference's expressions: the FP64 form has its own
+// (edge_end, erf_exp.h: refined quotients and roots, erf and exp from one table
+// step), multiply-adds of an expression are fused (-ffp-contract=on), and the
+// least-squares solve is applied edge by edge, through the Cramer weights of
+// each list (sum_j (G_k - G_i)*(c . (dels, delt, deln)) instead of the 3x3 solve
+// of the accumulated sums).
 //
 // A point is handled by a group of lanes, kFluxGroup = 4 of them unless the
 // points are few (flux_small), each taking every fourth neighbour, and the
 // group sums its partial residuals at the end, in an order that does not
 // depend on the number of lanes.  Per lane this is the same work as one lane
 // per point, but a resident wave holds 64 / kFluxGroup points instead of 64:
-// the neighbour data of all points in flight on one XCD then fits its 4 MB L2.  With one lane per point
-// at the 8 resident waves per CU the FP64 kernel's registers allow, each
-// point's q, qm and dq were fetched from HBM about 19 times per launch.
+// the neighbour data of all points in flight on one XCD then fits its 4 MB L2.
+// With one lane per point at the 8 resident waves per CU the FP64 kernel's
+// registers allow, each point's q, qm and dq were fetched from HBM about 19
+// times per launch.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -436,28 +439,48 @@ void launch_class(const DevGeom& g, const DevState& s, const FlowParams& p, cons
 
 }  // namespace
 
-// Launches both classes together where they do not fill the chip; false: they
-// take a launch each.  Four lanes take a point's 25 neighbours in seven steps
-// of some 7 us (FP64) each when a wave has its SIMD to itself, so with few
-// points the steps are what counts and more lanes share a point: 32 take one
-// step, 16 two.  They cost nothing while the chip has room, about a third more
-// than four lanes once it is full (the lanes beyond 25 idle, terms are moved
-// between lanes).  And the general class, an eighth of the points, leaves the
-// chip mostly idle by itself up to some 100,000 points, so it shares the
-// interior class's launch, until the interior class's registers (four waves
-// per SIMD in FP32 alone, three together) weigh more.  An iteration, in us,
-// with four lanes and a launch per class, and so (both with the library's
-// functions in FP64):
-//     1,090 points, FP64   142 ->  41     mixed   97 ->  34   (32 + 32 lanes)
-//    20,000                176 ->  89            114 ->  56   (32 + 16)
-//    50,000                204 -> 143            133 ->  91   (16 + 4)
-//   150,000                384 -> 336            229 -> 205   (4 + 4)
-//   500,000               1120 -> 1057           635 -> 625   (4 + 4)
-//   1,000,000 together    2197 -> 2132          1262 -> 1289: a launch each
+// Whether one launch takes both classes.  The general class, an eighth of the
+// points, leaves the chip mostly idle by itself up to some 100,000 points, and
+// in one launch it fills what the interior class leaves free.  The larger
+// registers of the two kernels then hold for both (FP32: three waves per SIMD
+// instead of the interior class's four), so the gain shrinks with the size.  An
+// explicit iteration in us, a launch per class -> one launch:
+//                       FP64            mixed
+//       1,209 points     87 ->   33      89 ->  31
+//      20,000           106 ->   62     105 ->  49
+//      50,000           137 ->  107     122 ->  84
+//     100,000           200 ->  178     174 -> 138
+//     170,000           290 ->  266     241 -> 217
+//     350,000           579 ->  545     458 -> 430
+//     500,000           816 ->  784     622 -> 610
+//     600,000           977 ->  949     746 -> 745  (best class shapes 735)
+//     750,000          1230 -> 1189     943 -> 937  (921)
+// The line, at 450,000 interior points, is where the mixed form's gain ends; it
+// serves both forms, and FP64 leaves 3% beyond it.  Below it no shape of a launch
+// per class is faster.  With weighted least squares at 150,000 points 246 -> 233
+// and 199 -> 183, at 170,000 (one launch 263 and 205) a launch each.
 bool flux_joint(const TypeLists& tl, double power) {
     const int ng = tl.n_fused_wall, ni = tl.n_fused_interior;
     return ng <= (power != 0.0 ? 20000 : 100000) && ni <= 450000;
 }
+
+// The joint launch, and the lanes that share a point in it; false: each class
+// takes a launch.  Four lanes take a point's 25 neighbours in seven steps, each
+// a chain of dependent loads and arithmetic, and with few points the steps are
+// what counts: 32 lanes take one step, 16 two.  They cost nothing while the chip
+// has room, about a third more than four lanes once it is full (the lanes beyond
+// 25 idle, terms are moved between lanes).  An iteration in us, FP64 / mixed, on
+// both sides of each line (general + interior lanes):
+//   general points 20,000   15,145 (100,000 in all)  16+4   178 / 138   4+4   172 / 145
+//                           22,592 (150,000)         16+4   245 / 194   4+4   240 / 199
+//   interior points 24,000  22,937 (27,000)          16+16   70 /  58   16+4   73 /  62
+//                           28,090 (33,000)          16+16   82 /  64   16+4   81 /  62
+//   general points 4,000     3,252 (20,000)          32+16   62 /  49   16+16  59 /  49
+//                            4,063 (27,000)          32+16   74 /  59   16+16  70 /  58
+//   interior points 4,000    3,777 (6,057)           32+32   39 /  34   32+16  41 /  34
+//                           16,748 (20,000)          32+32   64 /  50   32+16  62 /  49
+// and weighted, interior points 24,000: 23,760  16+16  69 / 62   16+4  67 / 57,
+// 29,040  84 / 74 and 73 / 60.
 template <typename T>
 static bool flux_small(const DevGeom& g, const DevState& s, const FlowParams& p, const TypeLists& tl,
                        hipStream_t st, int parts) {

@@ -1,13 +1,18 @@
-// kernels_fp64.hip -- FP64 kernels of the q-LSKUM pseudo-time iteration in
-// the reference's evaluation order.
+// kernels_fp64.hip -- the kernels of the q-LSKUM pseudo-time iteration beside
+// the fused flux and the sync-free sweeps.
 //
 // Streaming kernels take one thread per point; the gathering kernels a group
 // of lanes per point (q-derivatives: 4 lanes splitting conn; list-by-list
-// flux: one lane per direction list).  Every list-walking routine below
-// follows the reference routine named at it with the same association of
-// each product; the file is compiled with -ffp-contract=off.  The fused flux
-// kernels (kernels_flux_fused.hip) give the flux residual of every point
-// whose walk fits in 64 entries; this file keeps the list-by-list form for
+// flux: one lane per direction list).  The file is compiled with
+// -ffp-contract=off: nothing is fused that the source does not fuse.  The
+// conserved vector, the list-by-list flux, D_inv, the level sweeps and the state
+// update follow the reference routine named at them with the same association of
+// each product.  The q-derivatives and the time step do not, in any mode: they
+// split a point's neighbours over lanes, fuse multiply-adds explicitly, apply the
+// 3x3 inverse instead of Cramer's rule per component and take the time step from
+// a squared weight; the tests hold them to 1e-11 and 1e-13 of the reference's.
+// The fused flux kernels (kernels_flux_fused.hip) give the flux residual of every
+// point whose walk fits in 64 entries; this file keeps the list-by-list form for
 // the rest and for the reference-order mode.
 #include <hip/hip_runtime.h>
 
@@ -178,9 +183,9 @@ __global__ void __launch_bounds__(kBlock) k_timestep_den(DevGeom g, DevState s) 
 // What bounds it: its neighbour loads (7 per neighbour in FP64, 5 in the mixed
 // form), then the arithmetic of the loop and of the solve.  Multiply-adds are
 // fused, the solve takes the six cofactors once for all 15 derivatives, and
-// the FP64 form is compiled for two waves per SIMD: its 166 registers fit
-// three, where a cap at four waves spilled 24 of them into the loop.  2M
-// cloud, FP64: 881 -> 629 us.
+// the FP64 form is compiled for two waves per SIMD: its 158 registers fit three
+// (176 with weights: two), where a cap at four waves spilled 24 of them into the
+// loop.  2M cloud, FP64: 881 -> 629 us.
 constexpr int kQdGroup = 4;
 
 template <typename T>

@@ -2,8 +2,9 @@
 //
 // Every routine keeps the reference's expression order (Fortran a+b+c is
 // (a+b)+c, a*b*c is (a*b)*c) and kernels_fp64.hip is compiled with
-// -ffp-contract=off, so its only differences from the reference CPU build
-// come from the device exp/log/erf (ocml vs glibc, within an ulp or two).
+// -ffp-contract=off, so what it takes from here differs from the reference CPU
+// build only by the device exp/log/erf (ocml vs glibc, within an ulp or two);
+// its q-derivatives and time step are written apart, with fused multiply-adds.
 // The sync-free sweeps take the sweep form of the split fluxes (SWEEP below:
 // one refined quotient and root), the fused flux kernel its own forms
 // (kernels_flux_fused.hip), and both units -ffp-contract=on (a*b + c fused
