@@ -552,16 +552,19 @@ int build_plan(mfcfd_ctx* c, int form) {
     for (int m = 0; m < 2; ++m) c->sweep_chains.chain[m] = chain_for(resident[m], per_level);
     std::vector<int> slots[2][2];   // [direction][precision]
     std::vector<unsigned char> late_src[2][2];
-    {
-        std::vector<std::future<void>> work;
-        for (int dir = 0; dir < 2; ++dir)
-            for (int m = 0; m < 2; ++m)
-                if (c->sweep_chains.grouping(m) == m)
-                    work.push_back(std::async([&, dir, m] {
-                        group_positions(dir == 0 ? plan.fwd : plan.bwd, n, c->sweep_chains.chain[m], slots[dir][m],
-                                        late_src[dir][m]);
-                    }));
-        for (auto& w : work) w.get();
+    const SweepChains& chains = c->sweep_chains;
+    if (chains.grouping(0) >= 0 || chains.grouping(1) >= 0) {
+        auto group = [&](int dir) {
+            const SweepGrouper g(dir == 0 ? plan.fwd : plan.bwd, n);
+            auto cut = [&, dir](int m) { g.cut(chains.chain[m], slots[dir][m], late_src[dir][m]); };
+            std::future<void> mixed;
+            if (chains.grouping(1) == 1) mixed = std::async(cut, 1);
+            if (chains.grouping(0) == 0) cut(0);
+            if (mixed.valid()) mixed.get();
+        };
+        std::future<void> f = std::async(group, 0);
+        group(1);
+        f.get();
     }
     hipStream_t st = c->stream;
     c->sw_fwd.release();

@@ -248,47 +248,63 @@ int build_dir(const SweepPlanInputs& in, bool forward, SweepDirPlan& out) {
 
 }  // namespace
 
-void group_positions(const SweepDirPlan& plan, int n, int max_chain, std::vector<int>& slots,
-                     std::vector<unsigned char>& late_src) {
+SweepGrouper::SweepGrouper(const SweepDirPlan& p, int n) : plan(p), position(n, -1) {
     const int m = (int)plan.seq.size();
-    slots.clear();
-    late_src.assign(m, 0);
-    std::vector<int> at(n, -1);
-    for (int u = 0; u < m; ++u) at[plan.seq[u]] = u;
-    // height: the longest chain of dependents below a position; joins: the
-    // candidate of greatest height among those whose late dependency it is
-    std::vector<int> height(m, 0), joins(m, -1);
+    const int* seq = plan.seq.data();
+    const long long* ptr = plan.take_ptr.data();
+    const unsigned* take = plan.take.data();
+    int* at = position.data();
+    for (int u = 0; u < m; ++u) at[seq[u]] = u;
+    std::vector<int> height(m, 0);   // the longest chain of dependents below a position
     for (int u = m - 1; u >= 0; --u)
-        for (long long e = plan.take_ptr[u]; e < plan.take_ptr[u + 1]; ++e)
-            if (plan.take[e] & kTakeWait) {
-                int& h = height[at[plan.take[e] >> kTakeShift]];
+        for (long long e = ptr[u]; e < ptr[u + 1]; ++e)
+            if (take[e] & kTakeWait) {
+                int& h = height[at[take[e] >> kTakeShift]];
                 h = std::max(h, height[u] + 1);
             }
+    joins.assign(m, -1);
     for (int u = 0; u < m; ++u) {
         if (!plan.late[u]) continue;
-        int& j = joins[at[plan.take[plan.take_ptr[u + 1] - 1] >> kTakeShift]];
+        int& j = joins[at[take[ptr[u + 1] - 1] >> kTakeShift]];
         if (j < 0 || height[u] > height[j]) j = u;
     }
-    std::vector<char> placed(m, 0);
-    slots.reserve((size_t)m + kSweepGroup);
+}
+
+void SweepGrouper::cut(int max_chain, std::vector<int>& slots, std::vector<unsigned char>& late_src) const {
+    const int m = (int)plan.seq.size();
+    // raw pointers, and the groups written by index: stores of bytes would have
+    // every vector's own pointer read again
+    const long long* ptr = plan.take_ptr.data();
+    const unsigned* take = plan.take.data();
+    const int *at = position.data(), *next = joins.data();
+    late_src.assign(m, 0);
+    slots.assign(((size_t)m + kSweepGroup - 1) / kSweepGroup * kSweepGroup, -1);
+    int* slot = slots.data();
+    unsigned char* src = late_src.data();
+    std::vector<char> placed_positions(m, 0);
+    char* placed = placed_positions.data();
+    int k = 0;   // slots filled
     for (int u = 0; u < m; ++u) {
         if (placed[u]) continue;
         placed[u] = 1;
-        slots.push_back(u);
-        for (int tail = u, len = 1; len < max_chain && slots.size() % kSweepGroup != 0; ++len) {
-            const int v = joins[tail];
+        slot[k++] = u;
+        for (int tail = u, len = 1; len < max_chain && k % kSweepGroup != 0; ++len) {
+            const int v = next[tail];
             if (v < 0) break;
             bool ready = true;
-            for (long long e = plan.take_ptr[v]; e < plan.take_ptr[v + 1] && ready; ++e)
-                if (plan.take[e] & kTakeWait) ready = placed[at[plan.take[e] >> kTakeShift]];
+            for (long long e = ptr[v]; e < ptr[v + 1] && ready; ++e)
+                if (take[e] & kTakeWait) ready = placed[at[take[e] >> kTakeShift]];
             if (!ready) break;
             placed[v] = 1;
-            late_src[v] = (unsigned char)(1 + (slots.size() - 1) % kSweepGroup);
-            slots.push_back(v);
+            src[v] = (unsigned char)(1 + (k - 1) % kSweepGroup);
+            slot[k++] = v;
             tail = v;
         }
     }
-    while (slots.size() % kSweepGroup != 0) slots.push_back(-1);
+}
+
+void group_positions(SweepDirPlan& plan, int n, int max_chain) {
+    SweepGrouper(plan, n).cut(max_chain, plan.slots, plan.late_src);
 }
 
 int chain_for(int resident_waves, double per_level) {

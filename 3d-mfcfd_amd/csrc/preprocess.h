@@ -104,11 +104,21 @@ struct SweepPlan {
 // group therefore never waits for a later one, and inside it positions wait
 // only for earlier positions, so groups taken in order always finish,
 // however few of them run at a time.
-void group_positions(const SweepDirPlan& plan, int n, int max_chain, std::vector<int>& slots,
-                     std::vector<unsigned char>& late_src);
-inline void group_positions(SweepDirPlan& plan, int n, int max_chain) {
-    group_positions(plan, n, max_chain, plan.slots, plan.late_src);
-}
+void group_positions(SweepDirPlan& plan, int n, int max_chain);
+
+// The same for several chain lengths: what they share, and a cut for each.  The
+// plan outlives it; cuts may run side by side.
+class SweepGrouper {
+   public:
+    SweepGrouper(const SweepDirPlan& plan, int n);
+    void cut(int max_chain, std::vector<int>& slots, std::vector<unsigned char>& late_src) const;
+
+   private:
+    const SweepDirPlan& plan;
+    std::vector<int> position;  // [n] of each point (-1: none)
+    std::vector<int> joins;     // per position: of those whose late dependency it is, the one with the
+                                // longest chain of dependents (-1: none)
+};
 
 // Longest chain of positions a sweep workgroup hands from wave to wave, from
 // the waves resident on the chip and the plan's mean positions per dependency
